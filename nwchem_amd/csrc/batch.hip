@@ -162,12 +162,9 @@ int enqueue(Batch &B, int precision, const Plan &P) {
   const char *segs = (const char *)P.tab + n * asz;
   if (P.total > 0) {
     int rc;
-    if (mixed) {
-      bool sparse = false;
-      for (const Job *j : B.jobs) sparse = sparse || j->sparse;
+    if (mixed)
       rc = launch_fused_mixed((const MixedSegment *)segs, P.nseg, P.total, precision, P.grid,
-                              B.stream, sparse, sched_use(B.sched));
-    }
+                              B.stream, sched_use(B.sched));
     else if (P.choice.family == FAM_WG)
       rc = launch_fused_wg((const Segment *)segs, P.nseg, P.total, P.grid, B.stream);
     else

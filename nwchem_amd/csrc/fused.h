@@ -35,10 +35,11 @@
 
 namespace tce_t {
 
-// The 18 d1/d2 contractions of fused_mixed.hip in its pass order: kind
-// (0 = d2, 1 = d1), lone particle L (0 a, 1 b, 2 c), lone hole h (0 i, 1 j,
-// 2 k), sign (1 = minus).  The contraction index x (e of d2, m of d1) pairs
-// with L and the hole pair (r, s) = the two holes other than h on one
+// The 18 d1/d2 contractions of fused_mixed.hip in its pass order p = 6 L + 2
+// n + kind: kind (0 = d2, 1 = d1), lone particle L (0 a, 1 b, 2 c), lone hole
+// h (j, i, k for n = 0, 1, 2; 0 i, 1 j, 2 k), sign (1 = minus; the same for
+// the d2 and d1 of one (L, h)).  The contraction index x (e of d2, m of d1)
+// pairs with L and the hole pair (r, s) = the two holes other than h on one
 // operand (t(L e r s), <m L||r s>), so spin and irrep conservation of that
 // block fix x's spin to spin(r) + spin(s) - spin(L) and its irrep to
 // irrep(L) ^ irrep(r) ^ irrep(s).
@@ -46,28 +47,39 @@ struct PassDef {
   int kind, L, h, minus;
 };
 constexpr PassDef MIXED_PASS[18] = {
-    {0, 0, 2, 1},  // d2 N=1: -t(a e i j)<b c||k e>
-    {1, 0, 2, 1},  // d1 N=6: -t(b c k m)<m a||i j>
     {0, 0, 1, 0},  // d2 N=3: +t(a e i k)<b c||j e>
     {1, 0, 1, 0},  // d1 N=5: +t(b c j m)<m a||i k>
     {0, 0, 0, 1},  // d2 N=2: -t(a e j k)<b c||i e>
     {1, 0, 0, 1},  // d1 N=4: -t(b c i m)<m a||j k>
+    {0, 0, 2, 1},  // d2 N=1: -t(a e i j)<b c||k e>
+    {1, 0, 2, 1},  // d1 N=6: -t(b c k m)<m a||i j>
+    {0, 1, 1, 1},  // d2 N=6: -t(b e i k)<a c||j e>
+    {1, 1, 1, 1},  // d1 N=8: -t(a c j m)<m b||i k>
     {0, 1, 0, 0},  // d2 N=5: +t(b e j k)<a c||i e>
     {1, 1, 0, 0},  // d1 N=7: +t(a c i m)<m b||j k>
     {0, 1, 2, 0},  // d2 N=4: +t(b e i j)<a c||k e>
     {1, 1, 2, 0},  // d1 N=9: +t(a c k m)<m b||i j>
-    {0, 1, 1, 1},  // d2 N=6: -t(b e i k)<a c||j e>
-    {1, 1, 1, 1},  // d1 N=8: -t(a c j m)<m b||i k>
-    {0, 2, 2, 1},  // d2 N=7: -t(c e i j)<a b||k e>
-    {1, 2, 2, 1},  // d1 N=3: -t(a b k m)<m c||i j>
     {0, 2, 1, 0},  // d2 N=9: +t(c e i k)<a b||j e>
     {1, 2, 1, 0},  // d1 N=2: +t(a b j m)<m c||i k>
     {0, 2, 0, 1},  // d2 N=8: -t(c e j k)<a b||i e>
     {1, 2, 0, 1},  // d1 N=1: -t(a b i m)<m c||j k>
+    {0, 2, 2, 1},  // d2 N=7: -t(c e i j)<a b||k e>
+    {1, 2, 2, 1},  // d1 N=3: -t(a b k m)<m c||i j>
 };
+// bit 3 L + n: the sign of MIXED_PASS[6 L + 2 n]
+constexpr int mixed_minus() {
+  int m = 0;
+  for (int p = 0; p < 18; p += 2) m |= MIXED_PASS[p].minus << (p / 2);
+  return m;
+}
+constexpr int MIXED_MINUS = mixed_minus();
 // hole pair (r, s) of lone hole h
 constexpr int pair_r(int h) { return h == 0 ? 1 : 0; }
 constexpr int pair_s(int h) { return h == 2 ? 1 : 2; }
+
+// Equal boxes of a one-box task (TaskDev::eq): both holes or particles of
+// the pair are the same orbitals.
+enum { EQ_IJ = 1, EQ_JK = 2, EQ_AB = 4, EQ_BC = 8 };
 
 struct TaskDev {
   int op4, op5, op6;  // particle-space offsets of the task's particle tiles
@@ -82,6 +94,7 @@ struct TaskDev {
   // h7b / p7b tiles, ccsd_t_doubles_gpu.F:260-263, 924-927); outside it
   // every operand of the pass is zero.  x0 = x1 = 0: no orbital allowed.
   unsigned short x0[18], x1[18];
+  int eq;  // EQ_* of a one-box task whose boxes are equal, 0 otherwise
 };
 
 struct FusedArgs {
@@ -102,12 +115,13 @@ struct MixedArgs {
   const void *x2[3], *y2[3];  // d2: T2e, Vd2 (parts: FP32 | hi, lo | hi, mid, lo)
   const void *x1[3], *y1[3];  // d1: Wd1, T2m
   int Ek, Mk;
-  // Lambda-CCSD(T) passes (lambda.hip): the window of left-hand tiles of
-  // items [lam_item0, lam_item0 + window) read by the right-hand pass, and
-  // the Fock hole-particle block F[h][p] (or null) the left-hand pass adds.
-  const double *lam_y = nullptr, *lam_f = nullptr;
-  long lam_item0 = 0;
-  // CR-CCSD(T) right-hand pass: the denominator partials (2 per wave, as
+  // Pairs of jobs (Lambda- and CR-CCSD(T), lambda.hip), set in the right-hand
+  // job's arguments: the left-hand job's (device memory) and the spill slots
+  // of the workgroups (pair_slot_doubles each).
+  const MixedArgs *left = nullptr;
+  double *spill = nullptr;
+  const double *lam_f = nullptr;  // left-hand job: Fock hole-particle block F[h][p] or null
+  // CR-CCSD(T), right-hand job: the denominator partials (2 per wave, as
   // f.partials holds the moment partials).
   double *cr_den = nullptr;
 };
@@ -141,17 +155,7 @@ struct FusedArgsG {
   int no, nv, Ep, Mp;
   gptr<double> partials;
 };
-struct MixedArgsG {
-  FusedArgsG f;
-  gptr<const void> x2[3], y2[3];
-  gptr<const void> x1[3], y1[3];
-  int Ek, Mk;
-  gptr<const double> lam_y, lam_f;
-  long lam_item0;
-  gptr<double> cr_den;
-};
 static_assert(sizeof(FusedArgsG) == sizeof(FusedArgs), "argument mirror");
-static_assert(sizeof(MixedArgsG) == sizeof(MixedArgs), "argument mirror");
 
 __device__ __forceinline__ FusedArgsG load_args(const FusedArgs *p) {
   const gptr<const FusedArgs> q = (gptr<const FusedArgs>)p;
@@ -172,25 +176,6 @@ __device__ __forceinline__ FusedArgsG load_args(const FusedArgs *p) {
   A.Mp = q->Mp;
   A.partials = (gptr<double>)q->partials;
   return A;
-}
-
-__device__ __forceinline__ MixedArgsG load_args(const MixedArgs *p) {
-  const gptr<const MixedArgs> q = (gptr<const MixedArgs>)p;
-  MixedArgsG M;
-  M.f = load_args(&p->f);
-  for (int i = 0; i < 3; ++i) {
-    M.x2[i] = (gptr<const void>)q->x2[i];
-    M.y2[i] = (gptr<const void>)q->y2[i];
-    M.x1[i] = (gptr<const void>)q->x1[i];
-    M.y1[i] = (gptr<const void>)q->y1[i];
-  }
-  M.Ek = q->Ek;
-  M.Mk = q->Mk;
-  M.lam_y = (gptr<const double>)q->lam_y;
-  M.lam_f = (gptr<const double>)q->lam_f;
-  M.lam_item0 = q->lam_item0;
-  M.cr_den = (gptr<double>)q->cr_den;
-  return M;
 }
 
 // First item of workgroup b in a persistent launch of G workgroups.  The
@@ -267,8 +252,8 @@ __device__ __forceinline__ void sched_leave(unsigned long long *sched) {
 // per item replaces a binary search of the table.  An item taken from
 // another queue can lie before the previous one: the scan restarts.  Empty
 // segments are stepped over.
-template <class Args>
-__device__ __forceinline__ int next_segment(const SegmentT<Args> *segs, int nseg, int s, long g) {
+template <class Segs>
+__device__ __forceinline__ int next_segment(Segs segs, int nseg, int s, long g) {
   if (g < segs[s].g0) s = 0;
   while (s + 1 < nseg && segs[s + 1].g0 <= g) ++s;
   return s;
@@ -384,7 +369,8 @@ __device__ __forceinline__ void wave_sum(double &e4, double &e5) {
 // Locate the task of a work item (tasks sorted by item0, item0[t] >= t) --
 // uniform.  Sub-tiled tables have one item per task (item0[t] == t): one
 // probe finds it.
-__device__ __forceinline__ int find_task(gptr<const TaskDev> tasks, int ntasks, long item) {
+template <class Tasks>
+__device__ __forceinline__ int find_task(Tasks tasks, int ntasks, long item) {
   if (item < ntasks && tasks[item].item0 == item) return (int)item;
   int lo = 0, hi = ntasks - 1;
   while (lo < hi) {
@@ -401,33 +387,27 @@ __device__ __forceinline__ int find_task(gptr<const TaskDev> tasks, int ntasks, 
 // segments (device table), `grid` persistent workgroups.
 int launch_fused_wave(const Segment *segs, int nseg, long total, int grid, hipStream_t s);
 int launch_fused_wg(const Segment *segs, int nseg, long total, int grid, hipStream_t s);
-// sparse: some job of the table narrows its passes' contraction ranges
-// (TaskDev::x0/x1, spin- or irrep-labelled tiles).
 // sched: the stream's counters of the dynamic schedule (sched_alloc), or
 // null for the static round-robin.
 int launch_fused_mixed(const MixedSegment *segs, int nseg, long total, int precision, int grid,
-                       hipStream_t s, bool sparse, unsigned long long *sched);
+                       hipStream_t s, unsigned long long *sched);
 // One task's t3 tiles (fused_mixed.hip): `total` items of the single task at
 // args->f.tasks[0], tiles written to args->f.partials (doubles, then singles).
 int launch_fused_tiles(const MixedSegment *segs, long total, int precision, int grid,
-                       hipStream_t s, bool sparse, unsigned long long *sched);
-// The Lambda-CCSD(T) passes over one segment of a job's items (8-wide
-// boxes).  left = true: the left-hand job's doubles (plus the Fock term of
-// args->lam_f) and singles of each wave's 4096 elements, in register order,
-// into args->f.partials at window slot (item - lam_item0) * 8 + wave (8192
-// doubles per slot).  left = false: the right-hand job's energy partials
-// factor * t3d * (y3 doubles) / D and factor * t3d * (y3 doubles + singles)
-// / D with the left-hand values read from args->lam_y at the same slots.
-int launch_fused_lambda(const MixedSegment *segs, long total, int precision, int grid,
-                        hipStream_t s, bool sparse, unsigned long long *sched, bool left);
-// The CR-CCSD(T) right-hand pass (in `precision`): the right-hand job's t3 doubles
-// (the moment M3 of cr_ccsd_t_N) and singles (the denominator tile of
-// cr_ccsd_t_E) against the left-hand job's t3 doubles and singles in the
-// window at args->lam_y: per wave factor * M3 * td / D and factor * M3 *
-// (td + ts) / D into args->f.partials, the same with the denominator tile
-// into args->cr_den.
-int launch_fused_cr_right(const MixedSegment *segs, long total, int precision, int grid,
-                          hipStream_t s, bool sparse, unsigned long long *sched);
+                       hipStream_t s, unsigned long long *sched);
+// Lambda-CCSD(T) or CR-CCSD(T) over one segment of the right-hand job's items
+// (8-wide boxes): per item the contractions of args->left, then those of the
+// segment's job.  Lambda: factor * t3d * (y3 doubles) / D and factor * t3d *
+// (y3 doubles + singles) / D per wave into args->f.partials, the y3 doubles
+// with the Fock term of left->lam_f.  CR: the right-hand job's t3 doubles (the
+// moment M3 of cr_ccsd_t_N) and singles (the denominator tile of cr_ccsd_t_E)
+// against the left-hand job's t3 doubles td and singles ts: factor * M3 * td /
+// D and factor * M3 * (td + ts) / D into args->f.partials, the same with the
+// denominator tile into args->cr_den.
+int launch_fused_pair(const MixedSegment *segs, long total, int precision, int grid, hipStream_t s,
+                      unsigned long long *sched, bool cr);
+// Doubles of one workgroup's slot of MixedArgs::spill.
+constexpr long pair_slot_doubles(bool cr) { return cr ? 8L * 8192 : 8L * 4096; }
 // Zeroed counters of the dynamic schedule for one launching stream (every
 // launch leaves them zero; launches that may overlap need their own), or
 // null on failure (error set).  Free with hipFree.

@@ -48,7 +48,7 @@ struct Job {
   int grid = 0;
   int pbox = 4;  // particle box edge of a work item: 4 (fused_wave) or 8 (fused_wg)
   bool k16 = false;  // FP64 on the 16x16 MFMA kernel (fused_triples_mixed, FP64 policy)
-  bool sparse = false;  // some task's contraction ranges are narrower than the spaces
+  bool whole = false;  // contraction ranges span the whole spaces (TCE_T_SPARSE=0)
   int ppi = 1;   // energy partials per work item (waves per item)
   // reduced-precision path (fused_mixed.hip): 8-wide particle boxes always
   std::vector<TaskDev> tasks8;
@@ -61,6 +61,8 @@ struct Job {
   void *tab_host = nullptr, *tab_dev = nullptr;
   void *dtile = nullptr;  // tile export: task entry, then doubles and singles tiles
   size_t dtile_bytes = 0;
+  double *dspill = nullptr;  // spill slots of a pair's launches (lambda.hip)
+  size_t dspill_bytes = 0;
   struct Mixed {
     void *x2[3] = {nullptr, nullptr, nullptr}, *y2[3] = {nullptr, nullptr, nullptr};  // T2e, Vd2
     void *x1[3] = {nullptr, nullptr, nullptr}, *y1[3] = {nullptr, nullptr, nullptr};  // Wd1, T2m
@@ -97,7 +99,9 @@ int prepare_mixed(Job &J, int precision);
 // The arguments M and one segment of items [item0, item1) in the job's
 // launch table, copied on J.stream (the host staging is reused by the next
 // call: synchronise J.stream first); the device segment, or null.
-const MixedSegment *stage_mixed(Job &J, const MixedArgs &M, long item1, long item0);
+// With `left`, the left-hand job's arguments of a pair go along (M.left).
+const MixedSegment *stage_mixed(Job &J, MixedArgs M, long item1, long item0,
+                                const MixedArgs *left = nullptr);
 // Kernel arguments of a job: FP64 with the job's own task table (wide =
 // false) or the 8-wide one (wide = true); reduced precision.
 FusedArgs job_args(const Job &J, bool wide);

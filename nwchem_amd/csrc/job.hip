@@ -211,7 +211,8 @@ struct ClassRanges {
   // [lo, hi) per (space 0 = occupied / 1 = virtual, spin 0..3, irrep 0..7);
   // hi = 0: no orbital of that class
   long lo[2][4][8], hi[2][4][8];
-  explicit ClassRanges(const Tiles &T) {
+  bool whole;  // every range spans its space
+  ClassRanges(const Tiles &T, bool whole_) : whole(whole_) {
     for (int sp = 0; sp < 2; ++sp)
       for (int a = 0; a < 4; ++a)
         for (int g = 0; g < 8; ++g) lo[sp][a][g] = 0, hi[sp][a][g] = 0;
@@ -232,6 +233,10 @@ struct ClassRanges {
       const long spin = T.spn(r) + T.spn(s) - T.spn(L), sym = T.sy(L) ^ T.sy(r) ^ T.sy(s);
       const int sp = q.kind == 1 ? 0 : 1;
       const bool ok = spin >= 0 && spin <= 3 && sym >= 0 && sym <= 7;
+      if (whole) {
+        d.x0[p] = 0, d.x1[p] = (unsigned short)(sp ? T.nv : T.no);
+        continue;
+      }
       d.x0[p] = ok ? (unsigned short)lo[sp][spin][sym] : 0;
       d.x1[p] = ok ? (unsigned short)hi[sp][spin][sym] : 0;
     }
@@ -246,16 +251,58 @@ struct ClassRanges {
 // ccsd_t_gpu.F:153-167 applies them to tiles, so the reference task's energy
 // is the sum of its sub-tasks' and no symmetric duplicate is computed.
 // bound[t] = first item of reference task t (bound[ntask] = items).
-static long build_tasks(const Tiles &T, int pb, bool sub, std::vector<TaskDev> &tasks,
-                        std::vector<long> &bound, std::vector<long> *task_tiles) {
+//
+// One-box tasks (sub, or one_box: tiles that are boxes themselves) take their
+// particle boxes and their hole boxes in descending order of size: t3 t3 / D
+// and t3 y3 / D do not depend on the order, and fused_triples_mixed wastes no
+// MFMA on short second and third boxes (quads past an edge are skipped; the
+// first hole box is the MFMA row index and always counts 4).  TaskDev::eq
+// names the equal boxes.
+static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool whole,
+                        std::vector<TaskDev> &tasks, std::vector<long> &bound,
+                        std::vector<long> *task_tiles) {
   const long noab = T.noab, nvab = T.nvab;
   long item = 0;
   tasks.clear();
   bound.clear();
   if (task_tiles) task_tiles->clear();
-  const ClassRanges cr(T);
+  const ClassRanges cr(T, whole);
   struct Piece {
     int o, r;
+  };
+  // Order of three boxes by descending size (stable): position of each.
+  auto order3 = [](const Piece (&x)[3], int (&k)[3]) {
+    k[0] = 0, k[1] = 1, k[2] = 2;
+    if (x[0].r < x[1].r) std::swap(k[0], k[1]);
+    if (x[k[1]].r < x[k[2]].r) std::swap(k[1], k[2]);
+    if (x[k[0]].r < x[k[1]].r) std::swap(k[0], k[1]);
+  };
+  // Fills the boxes, their equalities and the contraction ranges of a one-box
+  // task of tiles t6; `have` caches the ranges by box order within a task.
+  struct Ranges {
+    bool set = false;
+    TaskDev d;
+  };
+  auto one_box_task = [&](TaskDev &d, const long (&t6)[6], const Piece (&p)[3],
+                          const Piece (&h)[3], std::vector<Ranges> &have) {
+    int kp[3], kh[3];
+    order3(p, kp);
+    order3(h, kh);
+    d.op4 = p[kp[0]].o, d.op5 = p[kp[1]].o, d.op6 = p[kp[2]].o;
+    d.oh1 = h[kh[0]].o, d.oh2 = h[kh[1]].o, d.oh3 = h[kh[2]].o;
+    d.r4 = p[kp[0]].r, d.r5 = p[kp[1]].r, d.r6 = p[kp[2]].r;
+    d.r1 = h[kh[0]].r, d.r2 = h[kh[1]].r, d.r3 = h[kh[2]].r;
+    d.nb4 = d.nb5 = d.nb6 = d.nb1 = d.nb2 = d.nb3 = 1;
+    d.eq = (d.oh1 == d.oh2 ? EQ_IJ : 0) | (d.oh2 == d.oh3 ? EQ_JK : 0) |
+           (d.op4 == d.op5 ? EQ_AB : 0) | (d.op5 == d.op6 ? EQ_BC : 0);
+    Ranges &r = have[(kp[0] * 3 + kp[1]) * 9 + kh[0] * 3 + kh[1]];
+    if (!r.set) {
+      const long t[6] = {t6[kp[0]], t6[kp[1]], t6[kp[2]], t6[3 + kh[0]], t6[3 + kh[1]], t6[3 + kh[2]]};
+      cr.set(T, t, r.d);
+      r.set = true;
+    }
+    std::copy(r.d.x0, r.d.x0 + 18, d.x0);
+    std::copy(r.d.x1, r.d.x1 + 18, d.x1);
   };
   // sub-tiles of tile b with edge e (the last one ragged)
   auto pieces = [&](long b, int e, bool hole) {
@@ -285,36 +332,37 @@ static long build_tasks(const Tiles &T, int pb, bool sub, std::vector<TaskDev> &
               if (!task_allowed(T, p4b, p5b, p6b, h1b, h2b, h3b)) continue;
               bound.push_back(item);
               const long tiles6[6] = {p4b, p5b, p6b, h1b, h2b, h3b};
-              TaskDev ranges;
-              cr.set(T, tiles6, ranges);
+              std::vector<Ranges> have(81);
               if (task_tiles) {
                 long tt[6] = {p4b, p5b, p6b, h1b, h2b, h3b};
                 task_tiles->insert(task_tiles->end(), tt, tt + 6);
               }
               if (!sub) {
                 TaskDev d;
-                d.op4 = (int)(T.ofs(p4b) - T.no);
-                d.op5 = (int)(T.ofs(p5b) - T.no);
-                d.op6 = (int)(T.ofs(p6b) - T.no);
-                d.oh1 = (int)T.ofs(h1b);
-                d.oh2 = (int)T.ofs(h2b);
-                d.oh3 = (int)T.ofs(h3b);
-                d.r4 = (int)T.rng(p4b);
-                d.r5 = (int)T.rng(p5b);
-                d.r6 = (int)T.rng(p6b);
-                d.r1 = (int)T.rng(h1b);
-                d.r2 = (int)T.rng(h2b);
-                d.r3 = (int)T.rng(h3b);
-                d.nb4 = (d.r4 + pb - 1) / pb;
-                d.nb5 = (d.r5 + pb - 1) / pb;
-                d.nb6 = (d.r6 + pb - 1) / pb;
-                d.nb1 = (d.r1 + 3) / 4;
-                d.nb2 = (d.r2 + 3) / 4;
-                d.nb3 = (d.r3 + 3) / 4;
+                const Piece p[3] = {{(int)(T.ofs(p4b) - T.no), (int)T.rng(p4b)},
+                                    {(int)(T.ofs(p5b) - T.no), (int)T.rng(p5b)},
+                                    {(int)(T.ofs(p6b) - T.no), (int)T.rng(p6b)}};
+                const Piece h[3] = {{(int)T.ofs(h1b), (int)T.rng(h1b)},
+                                    {(int)T.ofs(h2b), (int)T.rng(h2b)},
+                                    {(int)T.ofs(h3b), (int)T.rng(h3b)}};
+                if (one_box) {
+                  one_box_task(d, tiles6, p, h, have);
+                } else {
+                  d.op4 = p[0].o, d.op5 = p[1].o, d.op6 = p[2].o;
+                  d.oh1 = h[0].o, d.oh2 = h[1].o, d.oh3 = h[2].o;
+                  d.r4 = p[0].r, d.r5 = p[1].r, d.r6 = p[2].r;
+                  d.r1 = h[0].r, d.r2 = h[1].r, d.r3 = h[2].r;
+                  d.nb4 = (d.r4 + pb - 1) / pb;
+                  d.nb5 = (d.r5 + pb - 1) / pb;
+                  d.nb6 = (d.r6 + pb - 1) / pb;
+                  d.nb1 = (d.r1 + 3) / 4;
+                  d.nb2 = (d.r2 + 3) / 4;
+                  d.nb3 = (d.r3 + 3) / 4;
+                  d.eq = 0;
+                  cr.set(T, tiles6, d);
+                }
                 d.item0 = item;
                 d.factor = task_factor(T.restricted, p4b, p5b, p6b, h1b, h2b, h3b);
-                std::copy(ranges.x0, ranges.x0 + 18, d.x0);
-                std::copy(ranges.x1, ranges.x1 + 18, d.x1);
                 item += (long)d.nb4 * d.nb5 * d.nb6 * d.nb1 * d.nb2 * d.nb3;
                 tasks.push_back(d);
                 continue;
@@ -326,16 +374,11 @@ static long build_tasks(const Tiles &T, int pb, bool sub, std::vector<TaskDev> &
               const double rf = T.restricted ? 2.0 : 1.0;
               auto emit = [&](size_t a, size_t b, size_t c, size_t i, size_t j, size_t k) {
                 TaskDev d;
-                d.op4 = A[a].o, d.op5 = B[b].o, d.op6 = C[c].o;
-                d.oh1 = I[i].o, d.oh2 = J[j].o, d.oh3 = K[k].o;
-                d.r4 = A[a].r, d.r5 = B[b].r, d.r6 = C[c].r;
-                d.r1 = I[i].r, d.r2 = J[j].r, d.r3 = K[k].r;
-                d.nb4 = d.nb5 = d.nb6 = d.nb1 = d.nb2 = d.nb3 = 1;
+                const Piece p[3] = {A[a], B[b], C[c]}, h[3] = {I[i], J[j], K[k]};
+                one_box_task(d, tiles6, p, h, have);
                 d.item0 = item++;
                 d.factor = rf * sym_factor(hij && i == j, hjk && j == k) *
                            sym_factor(pab && a == b, pbc && b == c);
-                std::copy(ranges.x0, ranges.x0 + 18, d.x0);
-                std::copy(ranges.x1, ranges.x1 + 18, d.x1);
                 tasks.push_back(d);
               };
               if (holes_inner) {
@@ -397,11 +440,11 @@ static Tiles orbital_tiles(const Tiles &T, int ep) {
 // Kernel task table of a job in its tiling mode (pb: particle box).
 static long job_tasks(const Job &J, int pb, std::vector<TaskDev> &tasks, std::vector<long> &bound) {
   if (J.tiling == TCE_T_TILING_ORBITAL) {
-    const long n = build_tasks(orbital_tiles(J.T, pb), pb, false, tasks, bound, nullptr);
+    const long n = build_tasks(orbital_tiles(J.T, pb), pb, false, true, J.whole, tasks, bound, nullptr);
     bound.assign({0L, n});
     return n;
   }
-  return build_tasks(J.T, pb, J.tiling == TCE_T_TILING_SUBTILE, tasks, bound, nullptr);
+  return build_tasks(J.T, pb, J.tiling == TCE_T_TILING_SUBTILE, false, J.whole, tasks, bound, nullptr);
 }
 
 // Work items of a job's kernel tasks with pb-wide particle boxes (counted,
@@ -462,6 +505,8 @@ extern "C" int tce_t_job_create_tiling(const tce_t_tiles *tiles, int tiling, tce
   }
   auto J = std::make_unique<Job>();
   J->tiling = tiling;
+  if (const char *e = getenv("TCE_T_SPARSE"))  // 0: always the whole spaces
+    J->whole = !strcmp(e, "0");
   if (!J->T.load(tiles)) {
     set_error("invalid tile description");
     return TCE_T_ERR_ARG;
@@ -490,7 +535,7 @@ extern "C" int tce_t_job_create_tiling(const tce_t_tiles *tiles, int tiling, tce
   {  // the reference task list (per-task energies, restart blocks)
     std::vector<TaskDev> ref;
     std::vector<long> rb;
-    build_tasks(T, J->pbox, false, ref, rb, &J->task_tiles);
+    build_tasks(T, J->pbox, false, false, false, ref, rb, &J->task_tiles);
   }
   J->nitems = job_tasks(*J, J->pbox, J->tasks, J->bound);
   if (J->pbox == 8)
@@ -499,13 +544,6 @@ extern "C" int tce_t_job_create_tiling(const tce_t_tiles *tiles, int tiling, tce
     J->nitems8 = job_tasks(*J, 8, J->tasks8, J->bound8);
   J->Ep = round8(T.nv);
   J->Mp = round8(T.no);
-  for (const TaskDev &d : J->tasks8)
-    for (int p = 0; p < 18 && !J->sparse; ++p) {
-      const long full = MIXED_PASS[p].kind ? T.no : T.nv;
-      J->sparse = d.x0[p] > 0 || d.x1[p] < full;
-    }
-  if (const char *e = getenv("TCE_T_SPARSE"))  // 0: always the whole spaces
-    if (!strcmp(e, "0")) J->sparse = false;
   *out = reinterpret_cast<tce_t_job *>(J.release());
   return TCE_T_OK;
 }
@@ -543,7 +581,8 @@ extern "C" long tce_t_job_device_bytes(const tce_t_job *job) {
   if (!job) return -1;
   const Job &J = *reinterpret_cast<const Job *>(job);
   return dense_bytes(J) + J.nitems * J.ppi * 16 + (long)J.tasks.size() * sizeof(TaskDev) +
-         (J.ngroups() + 1) * 8 + J.ngroups() * 16 + 64 + (long)J.dtile_bytes;
+         (J.ngroups() + 1) * 8 + J.ngroups() * 16 + 64 + (long)J.dtile_bytes +
+         (long)J.dspill_bytes;
 }
 
 namespace {
@@ -873,8 +912,19 @@ static const SegmentT<Args> *stage_table(Job &J, const Args &args, long item1, l
   return (const SegmentT<Args> *)(d + off);
 }
 
-const MixedSegment *tce_t::stage_mixed(Job &J, const MixedArgs &M, long item1, long item0) {
+const MixedSegment *tce_t::stage_mixed(Job &J, MixedArgs M, long item1, long item0,
+                                       const MixedArgs *left) {
   if (ensure_table(J) != TCE_T_OK) return nullptr;
+  if (left) {
+    // in the second half of the table
+    constexpr size_t at = TAB_BYTES / 2;
+    static_assert((sizeof(MixedArgs) + 15) / 16 * 16 + sizeof(MixedSegment) <= at, "pair table");
+    std::memcpy((char *)J.tab_host + at, left, sizeof *left);
+    if (hipMemcpyAsync((char *)J.tab_dev + at, (char *)J.tab_host + at, sizeof *left,
+                       hipMemcpyHostToDevice, J.stream) != hipSuccess)
+      return nullptr;
+    M.left = (const MixedArgs *)((char *)J.tab_dev + at);
+  }
   return stage_table(J, M, item1, item0);
 }
 
@@ -1079,7 +1129,7 @@ extern "C" int tce_t_job_run(tce_t_job *job, int precision, double *e_bt, double
     if (!sg) return TCE_T_ERR_HIP;
     HIPCHK(hipEventRecord(J.ev0, J.stream), "event");
     lrc = launch_fused_mixed(sg, 1, J.nitems8, precision,
-                             (int)std::min<long>(std::max(1, cus), J.nitems8), J.stream, J.sparse,
+                             (int)std::min<long>(std::max(1, cus), J.nitems8), J.stream,
                              sched_use(J.dsched));
   } else {
     const long grid = std::min<long>(J.grid, J.nitems);
@@ -1174,7 +1224,7 @@ extern "C" int tce_t_job_run_restart(tce_t_job *job, int precision, long *begin,
         if (!sg) return TCE_T_ERR_HIP;
         lrc = launch_fused_mixed(sg, 1, i1 - i0, precision,
                                  (int)std::min<long>(std::max(1, cus), i1 - i0), J.stream,
-                                 J.sparse, sched_use(J.dsched));
+                                 sched_use(J.dsched));
       } else {
         const Segment *sg = stage_table(J, A, i1, i0);
         if (!sg) return TCE_T_ERR_HIP;
@@ -1275,7 +1325,7 @@ int tce_t::tile_export_device(Job &J, int precision, long h1b, long h2b, long h3
   d.factor = 1.0;
   {
     const long tiles6[6] = {p4b, p5b, p6b, h1b, h2b, h3b};
-    ClassRanges(T).set(T, tiles6, d);
+    ClassRanges(T, J.whole).set(T, tiles6, d);
   }
   const long n = (long)d.r1 * d.r2 * d.r3 * d.r4 * d.r5 * d.r6;
   const long items = (long)d.nb4 * d.nb5 * d.nb6 * d.nb1 * d.nb2 * d.nb3;
@@ -1316,7 +1366,7 @@ int tce_t::tile_export_device(Job &J, int precision, long h1b, long h2b, long h3
   int cus = 0;
   HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, J.device), "attr");
   if (launch_fused_tiles(sg, items, precision, (int)std::min<long>(std::max(1, cus), items),
-                         J.stream, J.sparse, sched_use(J.dsched)) != 0) {
+                         J.stream, sched_use(J.dsched)) != 0) {
     set_error("tile kernel launch failed");
     return TCE_T_ERR_HIP;
   }
@@ -1494,6 +1544,9 @@ void tce_t::job_release(Job &J) {
   if (J.dtile) (void)hipFree(J.dtile);
   J.dtile = nullptr;
   J.dtile_bytes = 0;
+  if (J.dspill) (void)hipFree(J.dspill);
+  J.dspill = nullptr;
+  J.dspill_bytes = 0;
   for (auto &m : J.mx) {
     for (int p = 0; p < 3; ++p)
       for (void **b : {&m.x2[p], &m.y2[p], &m.x1[p], &m.y1[p]}) {

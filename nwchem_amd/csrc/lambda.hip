@@ -162,14 +162,12 @@ int fock_hole_particle(const Tiles &T, const double *f1, const long *f1h,
 
 // Orbital pairing on the job's own kernel tasks (sub-tiles of the reference
 // tiles, each box once with its symmetry factor: the product t3 y3 / D is
-// symmetric under the permutations within equal tiles, as t3 t3 / D is).
-// The items run in windows of W: the left-hand pass leaves each item's y3
-// doubles (Fock term added) and singles in a window buffer in register
-// order, the right-hand pass forms the energy partials of the same items
-// from its t3 doubles and the window; the job's task reduction then gives
-// the per-task sums.  No tile leaves the registers in the tile layout.
-// cr_den (CR-CCSD(T)): the right-hand pass is the CR one; te gets the
-// moment sums, *te_den the denominator sums, per task.
+// symmetric under the permutations within equal tiles, as t3 t3 / D is): one
+// launch whose items run the left-hand job's contractions, then the right-hand
+// job's, and form the energy partials (launch_fused_pair); the job's task
+// reduction then gives the per-task sums.  No tile leaves the registers in the
+// tile layout.  cr_den (CR-CCSD(T)): the right-hand job is the CR one; te gets
+// the moment sums, *te_den the denominator sums, per task.
 int lambda_fused(Job &JR, Job &JL, const double *dF, int precision, std::vector<double> &te,
                  double *cr_den = nullptr, std::vector<double> *te_den = nullptr) {
   for (Job *J : {&JR, &JL}) {
@@ -182,52 +180,29 @@ int lambda_fused(Job &JR, Job &JL, const double *dF, int precision, std::vector<
     return TCE_T_ERR_ARG;
   }
   const long N = JR.nitems8, nt = JR.ntask();
-  constexpr long SLOT = 8L * 8192 * sizeof(double);  // window bytes per item (8 waves)
-  size_t free_b = 0, total_b = 0;
-  HIPCHK(hipMemGetInfo(&free_b, &total_b), "memory info");
-  const long budget = std::min<long>(16L << 30, (long)(free_b / 4));
-  long W = std::max(1L, std::min(N, budget / SLOT));
-  if (const char *w = getenv("TCE_T_LAMBDA_WINDOW")) {  // items per window (tests, tuning)
-    const long x = atol(w);
-    if (x > 0) W = std::min(W, x);
-  }
-  int cus = 0;
-  HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, JR.device), "attr");
-  double *win = nullptr;
-  HIPCHK(hipMalloc(&win, (size_t)W * SLOT), "lambda window");
   int rc = TCE_T_OK;
-  for (long i0 = 0; i0 < N && rc == TCE_T_OK; i0 += W) {
-    const long i1 = std::min(N, i0 + W);
-    const int grid = (int)std::min<long>(std::max(1, cus), i1 - i0);
-    MixedArgs ML = job_margs(JL, precision);
-    ML.f.partials = win;
+  if (N > 0) {
+    int cus = 0;
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, JR.device), "attr");
+    const int grid = (int)std::min<long>(std::max(1, cus), N);
+    const size_t need = (size_t)grid * pair_slot_doubles(cr_den != nullptr) * sizeof(double);
+    if (JR.dspill_bytes < need) {
+      if (JR.dspill) HIPCHK(hipFree(JR.dspill), "spill slots");
+      JR.dspill = nullptr;
+      JR.dspill_bytes = 0;
+      HIPCHK(hipMalloc(&JR.dspill, need), "spill slots");
+      JR.dspill_bytes = need;
+    }
+    MixedArgs ML = job_margs(JL, precision), MR = job_margs(JR, precision);
     ML.lam_f = dF;
-    ML.lam_item0 = i0;
-    const MixedSegment *sl = stage_mixed(JL, ML, i1, i0);
-    if (!sl || launch_fused_lambda(sl, i1 - i0, precision, grid, JL.stream, JL.sparse,
-                                   sched_use(JL.dsched), true) != 0) {
-      set_error("lambda left pass: launch failed");
-      rc = TCE_T_ERR_HIP;
-      break;
-    }
-    if (!hip_ok(hipStreamSynchronize(JL.stream), "lambda left pass")) {
-      rc = TCE_T_ERR_HIP;
-      break;
-    }
-    MixedArgs MR = job_margs(JR, precision);
-    MR.lam_y = win;
-    MR.lam_item0 = i0;
+    MR.spill = JR.dspill;
     MR.cr_den = cr_den;
-    const MixedSegment *sr = stage_mixed(JR, MR, i1, i0);
-    if (!sr || (cr_den ? launch_fused_cr_right(sr, i1 - i0, precision, grid, JR.stream, JR.sparse,
-                                               sched_use(JR.dsched))
-                       : launch_fused_lambda(sr, i1 - i0, precision, grid, JR.stream, JR.sparse,
-                                             sched_use(JR.dsched), false)) != 0) {
-      set_error("lambda right pass: launch failed");
+    const MixedSegment *sg = stage_mixed(JR, MR, N, 0, &ML);
+    if (!sg || launch_fused_pair(sg, N, precision, grid, JR.stream, sched_use(JR.dsched),
+                                 cr_den != nullptr) != 0) {
+      set_error("lambda launch failed");
       rc = TCE_T_ERR_HIP;
-      break;
     }
-    if (!hip_ok(hipStreamSynchronize(JR.stream), "lambda right pass")) rc = TCE_T_ERR_HIP;
   }
   // per-task sums of one partials buffer, in the order of the task list
   auto reduce = [&](const double *part, std::vector<double> &out) {
@@ -244,11 +219,7 @@ int lambda_fused(Job &JR, Job &JL, const double *dF, int precision, std::vector<
   };
   if (rc == TCE_T_OK) reduce(JR.dpart8, te);
   if (rc == TCE_T_OK && cr_den) reduce(cr_den, *te_den);
-  if (rc != TCE_T_OK) {  // nothing left in flight on either stream
-    (void)hipStreamSynchronize(JL.stream);
-    (void)hipStreamSynchronize(JR.stream);
-  }
-  (void)hipFree(win);
+  if (rc != TCE_T_OK) (void)hipStreamSynchronize(JR.stream);  // nothing left in flight
   return rc;
 }
 

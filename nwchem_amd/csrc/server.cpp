@@ -164,7 +164,6 @@ int run_slice(Server &S, int precision, const std::vector<Request *> &rs, float 
   // items per CU for each request)
   double total_cost = 0;
   long g = 0;
-  bool sparse = false;
   size_t ns = 0;  // segments: requests with items left (a system without
                   // allowed tasks has none and finishes without a launch)
   for (size_t k = 0; k < n; ++k) {
@@ -181,7 +180,6 @@ int run_slice(Server &S, int precision, const std::vector<Request *> &rs, float 
     take = std::max(1L, std::min(take, left));
     MixedArgs M = job_margs(J, precision);
     M.f.partials = r.dpart;
-    sparse = sparse || J.sparse;
     std::memcpy(h + ns * asz, &M, sizeof M);
     MixedSegment sg{(const MixedArgs *)(d + ns * asz), r.cursor, r.cursor + take, g};
     std::memcpy(h + n * asz + ns * ssz, &sg, sizeof sg);
@@ -198,7 +196,7 @@ int run_slice(Server &S, int precision, const std::vector<Request *> &rs, float 
   const int grid = (int)std::min<long>(S.cus, g);
   const int rc =
       launch_fused_mixed((const MixedSegment *)(d + n * asz), (int)ns, g, precision, grid, S.stream,
-                         sparse, sched_use(S.sched));
+                         sched_use(S.sched));
   if (rc != 0) {
     set_error("slice launch failed");
     return TCE_T_ERR_HIP;
