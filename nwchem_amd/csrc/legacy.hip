@@ -146,9 +146,8 @@ const int kD2L[9][6] = {{H3, H2, H1, P6, P5, P4}, {H2, H1, H3, P6, P5, P4}, {H2,
                         {H3, H2, H1, P4, P6, P5}, {H2, H1, H3, P4, P6, P5}, {H2, H3, H1, P4, P6, P5}};
 const int kD2S[9] = {-1, -1, +1, +1, +1, -1, -1, -1, +1};
 
-// One launch description: the output tile is walked in its own (layout)
-// order so stores are coalesced; every thread owns one t3 element and runs
-// the whole contraction for it.
+// One call: the output tile's extents and row codes in its own (layout)
+// order, operand strides by row code and the contraction.
 struct CallArgs {
   long dimL[6];   // extents in output order
   int codeL[6];   // row code at each output position
@@ -160,22 +159,105 @@ struct CallArgs {
   double sign;
 };
 
-__global__ void __launch_bounds__(256) contract_kernel(CallArgs c, double *__restrict__ t3,
+// The direct contraction.  Every variant's layout has the three hole indices
+// first (the block of F = h1 h2 h3 contiguous elements) and the three particle
+// indices after them, one to two of them on each operand.  A thread owns one
+// element of the hole block at TA x TB places of the particle indices, TA of
+// one that sits on the a operand and TB of one that sits on b: TA + TB operand
+// loads feed TA TB multiply-adds, and lanes read and write consecutive
+// elements of t3.
+// Bound: HBM, 16 bytes per element of t3 (read and written on each call; the
+// operands stay in L2), at tiles of 12^3 x 24^3 elements 82 us at the 4.7 TB/s
+// of a plain copy.  One element per thread, with two loads per multiply-add
+// and six 64-bit divisions per element, took 584 us per call on average.
+constexpr int TA = 4, TB = 4;
+struct DirectArgs {
+  unsigned F, d0, d1;          // hole block, its two fastest extents
+  long fa[3], fb[3];           // operand strides of the hole indices
+  int na, nb;                  // extents of the two tiled particle indices
+  unsigned tiles_a, tiles_b;   // tiles of them
+  long a_sa, b_sb;             // their operand strides
+  long a_t, b_t, c_t;          // strides of the particle indices in t3
+  long c_sa, c_sb;             // operand strides of the third one
+  unsigned threads, nc;        // per place of the third index; its extent
+  int K;
+  long ka, kb;
+  double sign;
+};
+
+DirectArgs direct_args(const CallArgs &c, int family) {
+  DirectArgs d;
+  long stride[6], s = 1;
+  for (int q = 0; q < 6; ++q) stride[q] = s, s *= c.dimL[q];
+  d.F = (unsigned)(c.dimL[0] * c.dimL[1] * c.dimL[2]);
+  d.d0 = (unsigned)c.dimL[0], d.d1 = (unsigned)c.dimL[1];
+  for (int q = 0; q < 3; ++q) d.fa[q] = c.sa[c.codeL[q]], d.fb[q] = c.sb[c.codeL[q]];
+  int qa = -1, qb = -1, qc = -1;
+  for (int q = 3; q < 6; ++q) {
+    const bool on_a = c.codeL[q] == P4 || (family == 1 && c.codeL[q] == P5);
+    if (on_a && qa < 0) qa = q;
+    else if (!on_a && qb < 0) qb = q;
+    else qc = q;
+  }
+  d.na = (int)c.dimL[qa], d.nb = (int)c.dimL[qb];
+  d.tiles_a = (unsigned)((d.na + TA - 1) / TA), d.tiles_b = (unsigned)((d.nb + TB - 1) / TB);
+  d.a_sa = c.sa[c.codeL[qa]], d.b_sb = c.sb[c.codeL[qb]];
+  d.a_t = stride[qa], d.b_t = stride[qb], d.c_t = stride[qc];
+  d.c_sa = c.sa[c.codeL[qc]], d.c_sb = c.sb[c.codeL[qc]];
+  d.threads = (unsigned)((long)d.F * d.tiles_a * d.tiles_b);
+  d.nc = (unsigned)c.dimL[qc];
+  d.K = (int)c.K;
+  d.ka = c.ka, d.kb = c.kb;
+  d.sign = c.sign;
+  return d;
+}
+
+__global__ void __launch_bounds__(256) contract_kernel(DirectArgs c, double *__restrict__ t3,
                                                        const double *__restrict__ a,
                                                        const double *__restrict__ b) {
-  long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= c.total) return;
-  long r = o, oa = 0, ob = 0;
+  const unsigned x = blockIdx.x * 256u + threadIdx.x;
+  if (x >= c.threads) return;
+  unsigned r = x / c.F;
+  const unsigned o = x - r * c.F;
+  const unsigned i0 = o % c.d0, i12 = o / c.d0, i1 = i12 % c.d1, i2 = i12 / c.d1;
+  const int pb = (int)(r % c.tiles_b) * TB;
+  r /= c.tiles_b;
+  const int pa = (int)r * TA;
+  const long pc = blockIdx.y;
+  const double *ap[TA], *bp[TB];
+  const long oa = i0 * c.fa[0] + i1 * c.fa[1] + i2 * c.fa[2] + pc * c.c_sa;
+  const long ob = i0 * c.fb[0] + i1 * c.fb[1] + i2 * c.fb[2] + pc * c.c_sb;
 #pragma unroll
-  for (int q = 0; q < 6; ++q) {
-    long v = r % c.dimL[q];
-    r /= c.dimL[q];
-    oa += v * c.sa[c.codeL[q]];
-    ob += v * c.sb[c.codeL[q]];
+  for (int u = 0; u < TA; ++u) ap[u] = a + oa + min(pa + u, c.na - 1) * c.a_sa;
+#pragma unroll
+  for (int v = 0; v < TB; ++v) bp[v] = b + ob + min(pb + v, c.nb - 1) * c.b_sb;
+  double *t = t3 + o + pa * c.a_t + pb * c.b_t + pc * c.c_t;
+  double old[TA][TB], acc[TA][TB];
+#pragma unroll
+  for (int u = 0; u < TA; ++u)
+#pragma unroll
+    for (int v = 0; v < TB; ++v) {
+      acc[u][v] = 0.0;
+      old[u][v] = pa + u < c.na && pb + v < c.nb ? t[u * c.a_t + v * c.b_t] : 0.0;
+    }
+#pragma unroll 2
+  for (int k = 0; k < c.K; ++k) {
+    double av[TA], bv[TB];
+#pragma unroll
+    for (int u = 0; u < TA; ++u) av[u] = ap[u][k * c.ka];
+#pragma unroll
+    for (int v = 0; v < TB; ++v) bv[v] = bp[v][k * c.kb];
+#pragma unroll
+    for (int u = 0; u < TA; ++u)
+#pragma unroll
+      for (int v = 0; v < TB; ++v) acc[u][v] = fma(av[u], bv[v], acc[u][v]);
   }
-  double acc = 0.0;
-  for (long k = 0; k < c.K; ++k) acc = fma(a[oa + k * c.ka], b[ob + k * c.kb], acc);
-  t3[o] += c.sign * acc;
+#pragma unroll
+  for (int u = 0; u < TA; ++u)
+#pragma unroll
+    for (int v = 0; v < TB; ++v)
+      if (pa + u < c.na && pb + v < c.nb)
+        t[u * c.a_t + v * c.b_t] = old[u][v] + c.sign * acc[u][v];
 }
 
 // TTGT back end (the alternative of sd_t_total_ttlg.cu: GEMM plus
@@ -339,8 +421,9 @@ void launch_call(int family, int n, const long dims[6], long K, const double *ha
                        t3, dC);
     if (!ok(hipGetLastError(), "permute_add_kernel launch")) return;
   } else {
-    hipLaunchKernelGGL(contract_kernel, dim3((unsigned)blocks), dim3(threads), 0, S.stream, c, t3,
-                       dops, dops + na);
+    const DirectArgs da = direct_args(c, family);
+    hipLaunchKernelGGL(contract_kernel, dim3((da.threads + 255) / 256, da.nc), dim3(256), 0,
+                       S.stream, da, t3, dops, dops + na);
     if (!ok(hipGetLastError(), "contract_kernel launch")) return;
   }
   if (host_t3 && !ok(hipMemcpyAsync(host_t3, t3, tbytes, hipMemcpyDeviceToHost, S.stream), "D2H t3"))
@@ -354,6 +437,11 @@ void launch_call(int family, int n, const long dims[6], long K, const double *ha
 // Energy of one task tile, layout (h3 fastest, h2, h1, p6, p5, p4 slowest)
 // as in ccsd_t_dot.F:89-110; first pass: one partial pair per block.  The
 // orbital energies of the six tiles are e1..e6 (h1, h2, h3, p4, p5, p6).
+// A unit of work is one particle triple by up to kEnChunk elements of its
+// hole block, whose e_h1 + e_h2 + e_h3 sit in LDS.
+// Bound: HBM, 16 bytes per element.  With five 64-bit divisions per element to
+// find its indices, 24e6 elements took 147 us; their bytes take 82 us.
+constexpr int kEnChunk = 2048;
 __device__ __forceinline__ void energy_block(long h1d, long h2d, long h3d, long p4d, long p5d,
                                              long p6d, const double *__restrict__ e1,
                                              const double *__restrict__ e2,
@@ -364,22 +452,33 @@ __device__ __forceinline__ void energy_block(long h1d, long h2d, long h3d, long 
                                              const double *__restrict__ t3d,
                                              const double *__restrict__ t3s,
                                              double *__restrict__ part) {
-  long total = h1d * h2d * h3d * p4d * p5d * p6d;
+  __shared__ double eh[kEnChunk];
+  const long F = h1d * h2d * h3d, P = p4d * p5d * p6d;
+  const long units = (F + kEnChunk - 1) / kEnChunk * P;
   double s1 = 0.0, s2 = 0.0;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (long)gridDim.x * blockDim.x) {
-    long r = i;
-    long h3 = r % h3d; r /= h3d;
-    long h2 = r % h2d; r /= h2d;
-    long h1 = r % h1d; r /= h1d;
-    long p6 = r % p6d; r /= p6d;
-    long p5 = r % p5d; r /= p5d;
-    long p4 = r;
-    double doub = t3d[i], sing = t3s[i];
-    double denom_0 = -(e4[p4] + e5[p5] + e6[p6]);
-    double denom = doub * factor / (e1[h1] + e2[h2] + e3[h3] + denom_0);
-    s1 += denom * doub;
-    s2 += denom * (doub + sing);
+  long cur = -1;
+  for (long u = blockIdx.x; u < units; u += gridDim.x) {
+    const long chunk = u / P, pt = u - chunk * P, f0 = chunk * kEnChunk;
+    const int n = (int)(F - f0 < kEnChunk ? F - f0 : kEnChunk);
+    if (chunk != cur) {  // uniform
+      __syncthreads();
+      for (int f = threadIdx.x; f < n; f += blockDim.x) {
+        const long x = f0 + f, r = x / h3d;
+        eh[f] = e1[r / h2d] + e2[r % h2d] + e3[x - r * h3d];
+      }
+      __syncthreads();
+      cur = chunk;
+    }
+    const long p45 = pt / p6d;
+    const double denom_0 = -(e4[p45 / p5d] + e5[p45 % p5d] + e6[pt - p45 * p6d]);
+    const double *d = t3d + pt * F + f0, *s = t3s + pt * F + f0;
+#pragma unroll 4
+    for (int f = threadIdx.x; f < n; f += 256) {
+      const double doub = d[f], sing = s[f];
+      const double denom = doub * factor / (eh[f] + denom_0);
+      s1 += denom * doub;
+      s2 += denom * (doub + sing);
+    }
   }
   __shared__ double r1[256], r2[256];
   r1[threadIdx.x] = s1;
@@ -430,16 +529,29 @@ constexpr int kEnThreads = 256;
 constexpr size_t kScratchDoubles = 2 * kEnBlocks;
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
-// Second pass: fixed-order sum of the block partials.
-__global__ void energy_final(const double *__restrict__ part, int nblk, double *__restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double a = 0.0, b = 0.0;
-    for (int i = 0; i < nblk; ++i) {
-      a += part[2 * i];
-      b += part[2 * i + 1];
+// Second pass: fixed-order sum of the block partials, one workgroup (one
+// thread over the 1024 pairs took 86 us, a chain of dependent loads and adds).
+__global__ void __launch_bounds__(256) energy_final(const double *__restrict__ part, int nblk,
+                                                    double *__restrict__ out) {
+  __shared__ double r1[256], r2[256];
+  double a = 0.0, b = 0.0;
+  for (int i = threadIdx.x; i < nblk; i += 256) {
+    a += part[2 * i];
+    b += part[2 * i + 1];
+  }
+  r1[threadIdx.x] = a;
+  r2[threadIdx.x] = b;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) {
+      r1[threadIdx.x] += r1[threadIdx.x + w];
+      r2[threadIdx.x] += r2[threadIdx.x + w];
     }
-    out[0] = a;
-    out[1] = b;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    out[0] = r1[0];
+    out[1] = r2[0];
   }
 }
 
@@ -617,7 +729,7 @@ extern "C" void compute_en_(double *factor, double *energy, double *eval1, doubl
   double *part = dbuf + ne, *out = part + 2 * nblk;
   hipLaunchKernelGGL(energy_partial, dim3(nblk), dim3(threads), 0, S.stream, d[0], d[1], d[2], d[3],
                      d[4], d[5], dbuf, *factor, S.t3_d, S.t3_s, part);
-  hipLaunchKernelGGL(energy_final, dim3(1), dim3(64), 0, S.stream, part, nblk, out);
+  hipLaunchKernelGGL(energy_final, dim3(1), dim3(kEnThreads), 0, S.stream, part, nblk, out);
   if (!ok(hipGetLastError(), "energy launch")) return;
   if (!ok(hipMemcpyAsync(S.pinned, out, 2 * sizeof(double), hipMemcpyDeviceToHost, S.stream), "D2H"))
     return;
@@ -689,7 +801,7 @@ extern "C" int tce_t_compute_en_noalloc(double factor, const double *t3d, const 
   hipLaunchKernelGGL(energy_partial_split, dim3(kEnBlocks), dim3(kEnThreads), 0, st, h1d, h2d, h3d,
                      p4d, p5d, p6d, eval1, eval2, eval3, eval4, eval5, eval6, factor, t3d, t3s,
                      part);
-  hipLaunchKernelGGL(energy_final, dim3(1), dim3(64), 0, st, part, kEnBlocks, energy);
+  hipLaunchKernelGGL(energy_final, dim3(1), dim3(kEnThreads), 0, st, part, kEnBlocks, energy);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error(std::string("tce_t_compute_en_noalloc launch: ") + hipGetErrorString(e));
