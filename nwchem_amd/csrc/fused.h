@@ -88,12 +88,13 @@ struct TaskDev {
   int nb4, nb5, nb6, nb1, nb2, nb3;  // boxes per index (particle box edge pbox, hole 4)
   long item0;                        // first work item of the task
   double factor;
-  // Contraction range of pass p of MIXED_PASS: orbitals [x0[p], x1[p]) of
+  // Contraction range of pass p of MIXED_PASS: orbitals [x0, x1) = [x[p] &
+  // 0xffff, x[p] >> 16) (one dword: scalar loads have no 16-bit form) of
   // the virtual (d2) or occupied (d1) space hold every orbital of the spin
   // and irrep the pass's blocks allow (the reference skips the other
   // h7b / p7b tiles, ccsd_t_doubles_gpu.F:260-263, 924-927); outside it
   // every operand of the pass is zero.  x0 = x1 = 0: no orbital allowed.
-  unsigned short x0[18], x1[18];
+  unsigned x[18];
   int eq;  // EQ_* of a one-box task whose boxes are equal, 0 otherwise
 };
 

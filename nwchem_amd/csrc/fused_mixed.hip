@@ -15,10 +15,16 @@
 //                 hi*mid, mid*hi, hi*lo, mid*mid, lo*hi), FP32 accumulation;
 //                 two LDS chunk buffers (three parts of 24 KB per chunk)
 //
-// Work item and workgroup as fused_wg.hip: one task x an 8x8x8 particle box x
-// a 4x4x4 hole box, 512 threads (8 waves, 2 per SIMD); a wave owns one 4x4x4
-// particle cube of the box by the hole box, 4096 t3 elements in 16 quads of
-// accumulators per lane.
+// Work item as fused_wg.hip: one task x an 8x8x8 particle box x a 4x4x4 hole
+// box; a wave owns one 4x4x4 particle cube of the box by the hole box, 4096 t3
+// elements in 16 quads of accumulators per lane.  A workgroup is 8 waves on
+// the whole item (split BF16) or 4 waves on one half of it along particle c
+// (FP64, FP32), two workgroups to a CU: while one waits at a chunk barrier, for
+// its first loads or in its epilogue, the other has the matrix cores.  With 8
+// waves in step, an FP64 item spent a quarter (no=40/nv=160) to two thirds
+// (short contraction ranges) of its time outside the MFMAs.  Half an item loads
+// 1.5 times the bytes per flop (8 to 10 of the L2's 64 bytes per clock and CU at
+// the FP64 rate); at the BF16 rate they would be most of that bandwidth.
 //
 // MFMA lane layout (16x16, probed on the device): A[i][k] at lane i+16(k/E),
 // B[k][j] at lane j+16(k/E) (E = k values per lane: 1 for f32, 8 for bf16),
@@ -90,8 +96,9 @@ struct Prec<TCE_T_FP64> {
   static constexpr int KC = 8;     // contraction values per chunk
   static constexpr int NPART = 1;  // operand parts
   static constexpr int ES = 8;     // bytes per element
+  static constexpr int NW = 4;     // waves of a workgroup
   // LDS chunk buffers (24 KB each), chunks loaded NBUF - 1 ahead
-  static constexpr int NBUF = 4;
+  static constexpr int NBUF = 3;
   typedef double acc;
   typedef d4 quad;
 };
@@ -100,6 +107,7 @@ struct Prec<TCE_T_FP32> {
   static constexpr int KC = 16;
   static constexpr int NPART = 1;
   static constexpr int ES = 4;
+  static constexpr int NW = 4;
   static constexpr int NBUF = 3;
   typedef float acc;
   typedef f4 quad;
@@ -109,6 +117,7 @@ struct Prec<TCE_T_BF16X3> {
   static constexpr int KC = 32;
   static constexpr int NPART = 2;  // hi, lo
   static constexpr int ES = 2;
+  static constexpr int NW = 8;
   static constexpr int NBUF = 3;
   typedef float acc;
   typedef f4 quad;
@@ -118,6 +127,7 @@ struct Prec<TCE_T_BF16X6> {
   static constexpr int KC = 32;
   static constexpr int NPART = 3;  // hi, mid, lo
   static constexpr int ES = 2;
+  static constexpr int NW = 8;
   static constexpr int NBUF = 2;   // 3 x 72 KB do not fit the 160 KB of LDS
   typedef float acc;
   typedef f4 quad;
@@ -171,8 +181,9 @@ struct HoleBox {
   int o, b0, rm, n;
 };
 __device__ __forceinline__ int hole(const HoleBox &h, int u) { return h.o + min(h.b0 + u, h.rm); }
-// Particle range of the box: global index g0 + min(slot, sm), slot = 0..7;
-// wave bit `bit` holds the wave's cube coordinate along it.
+// Particle range of the workgroup's box: global index g0 + min(slot, sm), slot =
+// 0..7 (0..3 of c in a half item); wave bit `bit` holds the wave's cube
+// coordinate along it.
 struct PRange {
   int g0, sm, bit;
 };
@@ -193,6 +204,11 @@ __device__ __forceinline__ PRange prange(const ItemGeo &G, int t) {
   return PRange{pick(G.a.g0, G.b.g0, G.c.g0), pick(G.a.sm, G.b.sm, G.c.sm),
                 pick(G.a.bit, G.b.bit, G.c.bit)};
 }
+// Slots of the second particle p2 of the pair beside lone particle L.
+template <int PREC>
+__device__ __forceinline__ int p2_slots(int L) {
+  return Prec<PREC>::NW == 4 && L != 2 ? 4 : 8;
+}
 // A wave's cube coordinate along a particle range.
 __device__ __forceinline__ int cube(int wave, const PRange &p) { return (wave >> p.bit) & 1; }
 
@@ -206,8 +222,12 @@ struct ItemPlan {
     return (h == 2 && (eq & EQ_IJ)) || (h == 0 && (eq & EQ_JK)) ? 1 : 0;
   }
 };
-__device__ __forceinline__ ItemPlan item_plan(int eq) {
+// half: a half item holds one c half, whose exchange with a or b needs the
+// other, so three equal particle boxes run as two there (the host's tables
+// put a pair of equal boxes on a and b).
+__device__ __forceinline__ ItemPlan item_plan(int eq, bool half) {
   ItemPlan P;
+  if (half && (eq & EQ_AB)) eq &= ~EQ_BC;
   P.eq = eq;
   const bool ij = eq & EQ_IJ, jk = eq & EQ_JK, ab = eq & EQ_AB, bc = eq & EQ_BC;
   P.hact = ij ? (jk ? 4 : 6) : (jk ? 3 : 7);  // k | j, k | i, j | all
@@ -231,12 +251,13 @@ __device__ __forceinline__ int x_swz(int slot, int r) {
 __device__ __forceinline__ int y_swz(int p1) { return (4 - (p1 & 3)) & 3; }
 
 // Direct global->LDS load of 16 bytes per lane: lane l writes LDS bytes
-// [m0 + 16 l, m0 + 16 l + 16).  Issued by inline assembly so that the
-// compiler does not tie later LDS reads of other buffers to it; the kernel
-// waits for these loads itself (vmcnt) before the barrier that publishes a
-// buffer.
-__device__ __forceinline__ void lds_load16(const void *g, unsigned lds_byte) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_byte), "v"(g)
+// [m0 + 16 l, m0 + 16 l + 16) from base + off.  Issued by inline assembly so
+// that the compiler does not tie later LDS reads of other buffers to it; the
+// kernel waits for these loads itself (vmcnt) before the barrier that publishes
+// a buffer.  Scalar base and LDS address: a load takes no VALU instruction.
+__device__ __forceinline__ void lds_load16(const char *base, unsigned off, unsigned lds_byte) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte), "v"(off),
+               "s"(base)
                : "memory");
 }
 // s_waitcnt vmcnt(N) with the other counters left alone (gfx9 encoding).
@@ -244,8 +265,8 @@ template <int N>
 __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
-// The same for a uniform n in 0..6 (a wave's loads of at most two chunks in
-// FP64, of one otherwise).
+// The same for a uniform n in 0..6 (a wave's loads of one chunk; 6 terms: up to
+// 9, waited for in full).
 __device__ __forceinline__ void wait_vm_n(int n) {
   switch (n) {
     case 6: wait_vm<6>(); break;
@@ -268,32 +289,46 @@ __device__ __forceinline__ void block_barrier() {
 template <int PREC>
 __device__ __forceinline__ int2 chunks_of(cptr<TaskDev> T, int p) {
   constexpr int KC = Prec<PREC>::KC;
-  const int x0 = T->x0[p], x1 = T->x1[p];
+  const unsigned x = T->x[p];
+  const int x0 = (int)(x & 0xffffu), x1 = (int)(x >> 16);
   const int c0 = x0 / KC;
   return make_int2(c0, x1 > x0 ? (x1 + KC - 1) / KC - c0 : 0);
 }
 
 // The loads of an item's chunk sequence: segments p = 6 L + 2 {j, i, k} +
-// {d2, d1} of MIXED_PASS with act's bit set, in order.  A thread loads up to
-// three quads of a chunk per operand part: the X quad of LDS block `wave`
-// (s-index wave >> 1, slots 4 (wave & 1) + lane >> 4) and the Y quads of
-// blocks 2 wave + t (h-index wave >> 1, p1 slots 4 (wave & 1) + 2t + lane >>
-// 5); blocks whose rows no quad of the pass reads are skipped (nl = loads per
-// chunk of this wave).
+// {d2, d1} of MIXED_PASS with act's bit set, in order.  A wave loads the X
+// blocks of s-index g (64 quads, 4 L slots each) and the Y blocks of h-index g
+// (64 quads, 16 particle pairs each), per operand part: with 8 waves g = wave
+// >> 1 and the waves of a pair take half of the L slots and p1 slots each, with
+// 4 waves g = wave.  Blocks whose rows no quad of the pass reads are skipped
+// (nl = loads per chunk of this wave).
 template <int PREC>
 struct Loader {
   using Pr = Prec<PREC>;
-  unsigned long xo, yo0, yo1;                 // the lane's row offsets (bytes)
-  const char *xb[Pr::NPART], *yb[Pr::NPART];  // tensors at the next chunk
+  static constexpr bool HALF = Pr::NW == 4;
+  static constexpr int NX = HALF ? 2 : 1, NY = HALF ? 4 : 2;
+  // The lane's rows relative to the first one of the box (bytes; 32 bits hold
+  // them in any tensor that fits the memory: three occupied indices of X,
+  // eight virtual ones of Y) and the tensors at that row and the next chunk.
+  unsigned xo[NX], yo[NY];
+  const char *xb[Pr::NPART], *yb[Pr::NPART];
   unsigned act;
   int p, left;  // segment (-1: none yet) and its chunks not yet loaded
-  bool lx, ly0, ly1;
+  unsigned on;  // bits 0..: X blocks loaded; bits 8..: Y blocks
   int nl;
+  int no, nv;         // extents of the job
+  unsigned rowe, rowm;  // bytes of a d2 and a d1 row
 
+  __device__ __forceinline__ void init(cptr<MixedArgs> A) {
+    p = -1;
+    left = 0;
+    no = A->f.no, nv = A->f.nv;
+    rowe = (unsigned)(A->Ek * Pr::ES), rowm = (unsigned)(A->Mk * Pr::ES);
+  }
   __device__ __forceinline__ void next_segment(cptr<MixedArgs> A, cptr<TaskDev> T,
                                                const ItemGeo &G, const ItemPlan &P, int wave,
                                                int lane_) {
-    constexpr int QE = 16 / Pr::ES;  // elements per quad
+    constexpr int QB = 16;  // bytes per quad
     const int lane = again(lane_);
     p = __builtin_ctz(act & (~0u << (p + 1)));
     const int L = p / 6, hi = (p >> 1) % 3, kind = p & 1;
@@ -303,46 +338,53 @@ struct Loader {
     const PRange PL = prange(G, L), P1 = prange(G, L == 0 ? 1 : 0), P2 = prange(G, L == 2 ? 1 : 2);
     const int2 ch = chunks_of<PREC>(T, p);
     left = ch.y;
-    const int no = A->f.no, nv = A->f.nv;
-    const unsigned row = (unsigned)((kind ? A->Mk : A->Ek) * Pr::ES);  // bytes
-    const long k0 = (long)ch.x * Pr::KC * Pr::ES;
+    const unsigned row = kind ? rowm : rowe;
+    const int g = HALF ? wave : wave >> 1;
+    const int r0 = hole(R, 0), hs = hole(S, g), hy = hole(H, g);
+    const unsigned k0 = (unsigned)(ch.x * Pr::KC * Pr::ES);
+    const long x0 = (long)(unsigned)((r0 * no + hs) * nv + PL.g0) * row + k0,
+               y0 = (long)(unsigned)((hy * nv + P1.g0) * nv + P2.g0) * row + k0;
 #pragma unroll
     for (int part = 0; part < Pr::NPART; ++part) {
-      xb[part] = (const char *)(kind ? A->x1[part] : A->x2[part]) + k0;
-      yb[part] = (const char *)(kind ? A->y1[part] : A->y2[part]) + k0;
+      xb[part] = (const char *)(kind ? A->x1[part] : A->x2[part]) + x0;
+      yb[part] = (const char *)(kind ? A->y1[part] : A->y2[part]) + y0;
     }
-    const int g = wave >> 1, half = 4 * (wave & 1);
-    lx = g >= P.s0(h) && g < S.n && half <= PL.sm;
-    ly0 = g < H.n && half <= P1.sm;
-    ly1 = g < H.n && half + 2 <= P1.sm;
-    nl = Pr::NPART * ((lx ? 1 : 0) + (ly0 ? 1 : 0) + (ly1 ? 1 : 0));
-    const int slot = half + (lane >> 4), xr = (lane >> 2) & 3;
-    const unsigned xrow = (unsigned)((hole(R, xr) * no + hole(S, g)) * nv + particle(PL, slot));
-    xo = (unsigned long)xrow * row + (unsigned)(QE * Pr::ES * ((lane & 3) ^ x_swz<PREC>(slot, xr)));
-    const int p2 = particle(P2, (lane >> 2) & 7), hy = hole(H, g);
+    on = 0;
+    nl = 0;
+    const int xr = (lane >> 2) & 3, kq = lane & 3;
+    const unsigned xrow = (unsigned)((hole(R, xr) - r0) * no * nv);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int s1 = half + 2 * t + (lane >> 5);
-      const unsigned yrow = (unsigned)((hy * nv + particle(P1, s1)) * nv + p2);
-      const unsigned long o =
-          (unsigned long)yrow * row + (unsigned)(QE * Pr::ES * ((lane & 3) ^ y_swz(s1)));
-      if (t == 0) yo0 = o;
-      else yo1 = o;
+    for (int u = 0; u < NX; ++u) {
+      const int first = HALF ? 4 * u : 4 * (wave & 1), slot = first + (lane >> 4);
+      if (g >= P.s0(h) && g < S.n && first <= PL.sm) on |= 1u << u, nl += Pr::NPART;
+      xo[u] = (xrow + min(slot, PL.sm)) * row + (unsigned)(QB * (kq ^ x_swz<PREC>(slot, xr)));
+    }
+    const bool wide = p2_slots<PREC>(L) == 8;  // rows of 8 p2 slots: 2 p1 slots to a block
+    const int p2 = min(wide ? (lane >> 2) & 7 : (lane >> 2) & 3, P2.sm);
+#pragma unroll
+    for (int t = 0; t < NY; ++t) {
+      const int first = HALF ? (wide ? 2 * t : 4 * t) : 4 * (wave & 1) + 2 * t;
+      const int s1 = first + (wide ? lane >> 5 : lane >> 4);
+      if (g < H.n && first <= P1.sm && (wide || t < 2)) on |= 256u << t, nl += Pr::NPART;
+      yo[t] = (unsigned)(min(s1, P1.sm) * nv + p2) * row + (unsigned)(QB * (kq ^ y_swz(s1)));
     }
   }
-  // The loads of the next chunk, into buffer b; returns their number.
+  // The loads of the next chunk into the buffer at LDS byte `base`; returns
+  // their number.  (Spread over the chunk's MFMAs, one block after each row of
+  // quads, they ran 1 to 2% slower than together.)
   __device__ __forceinline__ int load(cptr<MixedArgs> A, cptr<TaskDev> T, const ItemGeo &G,
-                                      const ItemPlan &P, unsigned lds_base, int b, int wave,
-                                      int lane) {
+                                      const ItemPlan &P, unsigned base, int wave, int lane) {
     if (left == 0) next_segment(A, T, G, P, wave, lane);
 #pragma unroll
     for (int part = 0; part < Pr::NPART; ++part) {
-      const unsigned base =
-          lds_base + (unsigned)(b * buf_quads<PREC>() + part * PART_QUADS) * 16u;
-      if (lx) lds_load16(xb[part] + xo, uniform((int)(base + wave * 1024u)));
-      const unsigned yl = base + X_QUADS * 16u + 2 * wave * 1024u;
-      if (ly0) lds_load16(yb[part] + yo0, uniform((int)yl));
-      if (ly1) lds_load16(yb[part] + yo1, uniform((int)(yl + 1024u)));
+      const unsigned b = base + part * PART_QUADS * 16u;
+#pragma unroll
+      for (int u = 0; u < NX; ++u)
+        if (on >> u & 1) lds_load16(xb[part], xo[u], b + (NX * wave + u) * 1024u);
+#pragma unroll
+      for (int t = 0; t < NY; ++t)
+        if (on >> (8 + t) & 1)
+          lds_load16(yb[part], yo[t], b + X_QUADS * 16u + (NY * wave + t) * 1024u);
       xb[part] += Pr::KC * Pr::ES;
       yb[part] += Pr::KC * Pr::ES;
     }
@@ -431,7 +473,7 @@ __device__ __forceinline__ int2 frag_offsets(const ItemGeo &G, int L, int wave, 
   const int p1s = 4 * cube(wave, prange(G, L == 0 ? 1 : 0)) + hi,
             p2s = 4 * cube(wave, prange(G, L == 2 ? 1 : 2)) + lo;
   return make_int2((slot * 4 + xr) * 4 + (kq ^ x_swz<PREC>(slot, xr)),
-                   (p1s * 8 + p2s) * 4 + (kq ^ y_swz(p1s)));
+                   (p1s * p2_slots<PREC>(L) + p2s) * 4 + (kq ^ y_swz(p1s)));
 }
 
 __device__ __forceinline__ float bperm(float v, int src) {
@@ -484,7 +526,6 @@ struct Stream {
   int todo;   // chunks of the item not yet loaded
   int ready;  // chunks not yet contracted
   int buf;    // buffer of the next chunk to contract
-  int pend;   // loads of the chunk after it still to be waited for (NBUF = 4)
 };
 
 // The chunks of one (L, h): X quads s0..s1-1 and Y quads 0..h1-1 (none in a
@@ -509,6 +550,8 @@ __device__ __forceinline__ void chunk_loop(typename Prec<PREC>::quad (&q)[16], c
     const f4 *cb = lds + st.buf * buf_quads<PREC>();
     int nl = 0;
     const int nb = st.buf + AH < NB ? st.buf + AH : st.buf + AH - NB;
+    const unsigned nbase = lds_base + (unsigned)nb * (buf_quads<PREC>() * 16u);
+    const bool more = st.todo > 0;
     // the MFMAs of X quad s
     auto row = [&](int s) {
       if (s < s0 || s >= s1) return;
@@ -534,27 +577,24 @@ __device__ __forceinline__ void chunk_loop(typename Prec<PREC>::quad (&q)[16], c
       row(0);
       row(1);
     }
-    if constexpr (NB >= 3)
-      if (st.todo > 0) {
-        nl = st.ld.load(A, T, G, P, lds_base, nb, wave, lane);
-        --st.todo;
-      }
+    if (NB >= 3 && more) {
+      nl = st.ld.load(A, T, G, P, nbase, wave, lane);
+      --st.todo;
+    }
     if (s1 > 0) {
       row(2);
       row(3);
     }
     // chunk j+1 landed once at most the loads of the later ones are pending
-    if constexpr (NB == 4) wait_vm_n(st.pend + nl);
-    else if constexpr (NB == 3) wait_vm_n(nl);
+    if constexpr (NB == 3) wait_vm_n(nl);
     else wait_vm<0>();
     block_barrier();
     if constexpr (NB == 2) {
-      if (st.todo > 0) {
-        st.ld.load(A, T, G, P, lds_base, st.buf, wave, lane);
+      if (more) {
+        st.ld.load(A, T, G, P, lds_base + (unsigned)st.buf * (buf_quads<PREC>() * 16u), wave, lane);
         --st.todo;
       }
     }
-    st.pend = nl;
     st.buf = st.buf + 1 < NB ? st.buf + 1 : 0;
   }
 }
@@ -562,13 +602,13 @@ __device__ __forceinline__ void chunk_loop(typename Prec<PREC>::quad (&q)[16], c
 // Subtracts the partner elements from the accumulators: with x' the element
 // of the exchanged particles (two exchanges when all boxes are equal), q =
 // q - q(a <-> b), q - q(b <-> c), or q - q(a <-> c) - q(b <-> c).  Through LDS
-// in rounds of 64 KB.  Layout c: lane = 4a' + b' + 16c'.
+// in rounds of 64 KB.  A half item has equal boxes a and b only.  Layout c: lane = 4a' + b' + 16c'.
 template <int PREC>
 __device__ __forceinline__ void exchange_particles(typename Prec<PREC>::quad (&q)[16], f4 *lds,
                                                    const ItemGeo &G, int eq, int wave, int lane_) {
   const int lane = again(lane_);
   constexpr int U = sizeof(typename Prec<PREC>::quad) / 16;  // 16-byte units per quad
-  constexpr int NQ = 8 / U;                                   // quads per round
+  constexpr int NQ = 64 / Prec<PREC>::NW / U;                 // quads per round
   const int a = (lane & 15) >> 2, b = lane & 3, c = lane >> 4;
   const int ca = cube(wave, G.a), cb = cube(wave, G.b), cc = cube(wave, G.c);
   auto from = [&](int x, int y, int z) { return (x << G.a.bit) | (y << G.b.bit) | (z << G.c.bit); };
@@ -672,24 +712,20 @@ __device__ __forceinline__ void contract(typename Prec<PREC>::quad (&q)[16], f4 
     st.ld.act |= on ? 1u << p : 0u;
     st.todo += on ? n : 0;
   }
-  st.ld.p = -1;
-  st.ld.left = 0;
+  st.ld.init(A);
   st.buf = 0;
-  {  // the first NBUF - 1 (two buffers: 2) chunks; the first one landed
-    constexpr int PRO = Pr::NBUF > 2 ? Pr::NBUF - 1 : 2;
-    int last = 0, before = 0;
+  {  // the first two chunks; the first one landed
+    int last = 0;
 #pragma unroll 1
-    for (int k = 0; k < PRO; ++k) {
-      before = last;
+    for (int k = 0; k < 2; ++k) {
       last = 0;
       if (st.todo > 0) {
-        last = st.ld.load(A, T, G, P, lds_base, k, wave, lane);
+        last = st.ld.load(A, T, G, P, lds_base + (unsigned)k * (buf_quads<PREC>() * 16u), wave, lane);
         --st.todo;
       }
     }
-    wait_vm_n(Pr::NBUF == 4 ? before + last : last);
+    wait_vm_n(last);
     block_barrier();
-    st.pend = last;
   }
   const bool live = 4 * cube(wave, G.a) <= G.a.sm && 4 * cube(wave, G.b) <= G.b.sm &&
                     4 * cube(wave, G.c) <= G.c.sm;
@@ -742,39 +778,52 @@ __device__ __forceinline__ void contract(typename Prec<PREC>::quad (&q)[16], f4 
 }
 
 // Stage the item's singles operands into LDS (FP64, as fused_wg.hip): 64 S
-// values (one hole pair, one particle pair) per wave and step; the pairs past
-// a ragged edge of the hole boxes are left out.
-__device__ __forceinline__ void stage_epilogue(double *e, cptr<FusedArgs> A, int wave, int lane_,
-                                               const ItemGeo &G) {
+// values of one hole pair per wave and load; the pairs past a ragged edge of
+// the hole boxes are left out.
+// Of the pairs (h, h') and (p, p') of an item: S[h][h'][p][p'] with rows of ld
+// elements, and T1 with element (p, h) at p * ldp + h * ldh.
+template <int NW>
+__device__ __forceinline__ void stage_epilogue(double *e, gptr<const double> S, int ld,
+                                               gptr<const double> T1, int ldp, int ldh, int no,
+                                               int nv, int wave, int lane_, const ItemGeo &G) {
   const int lane = again(lane_);
-  const int no = A->no, nv = A->nv;
-  const gptr<const double> S = (gptr<const double>)A->S, T1 = (gptr<const double>)A->T1;
-  const int p1 = lane >> 3, p2 = lane & 7;
+  // step 0, 1, 2: particle pair (b,c), (a,c), (a,b), 8 x 8 slots; a half item:
+  // (b,c) and (a,c) with 4 c slots in one step, then (a,b)
+  constexpr int STEPS = NW == 4 ? 2 : 3, R = 48 / NW;
 #pragma unroll
-  for (int sp = 0; sp < 3; ++sp) {
-    // wave w: hole pairs tp = w, w + 8, .. of this particle pair
-    const int g1 = particle(prange(G, sp == 0 ? 1 : 0), p1),
-              g2 = particle(prange(G, sp == 2 ? 1 : 2), p2);
-    double v[6];
+  for (int step = 0; step < STEPS; ++step) {
+    const bool both = NW == 4 && step == 0;
+    const int sp = both ? lane >> 5 : (NW == 4 ? 2 : step);
+    const int p1 = both ? (lane >> 2) & 7 : lane >> 3, p2 = both ? lane & 3 : lane & 7;
+    const int ga = particle(G.a, p1), gb = particle(G.b, p1);
+    const int g1 = sp == 0 ? gb : ga, g2 = particle(prange(G, step == STEPS - 1 ? 1 : 2), p2);
+    double v[R];
+    // wave w: hole pairs tp = w, w + NW, ..
 #pragma unroll
-    for (int r = 0; r < 6; ++r) {
-      const int tp = wave + 8 * r, t = r >> 1, u = (tp >> 2) & 3, w = tp & 3;
+    for (int r = 0; r < R; ++r) {
+      const int tp = wave + NW * r, t = (NW * r) >> 4, u = (tp >> 2) & 3, w = tp & 3;
       const HoleBox H1 = hole_box(G, t == 0 ? 1 : 0), H2 = hole_box(G, t == 2 ? 1 : 2);
       v[r] = 0.0;
       if (u < H1.n && w < H2.n)
-        v[r] = S[(unsigned long)(unsigned)((hole(H1, u) * no + hole(H2, w)) * nv + g1) * nv + g2];
+        v[r] = S[(unsigned long)(unsigned)((hole(H1, u) * no + hole(H2, w)) * nv + g1) * ld + g2];
     }
 #pragma unroll
-    for (int r = 0; r < 6; ++r) e[((wave + 8 * r) * 3 + sp) * 64 + lane] = v[r];
+    for (int r = 0; r < R; ++r) e[((wave + NW * r) * 3 + sp) * 64 + p1 * 8 + p2] = v[r];
   }
-  const int tid = wave * 64 + lane;
-  if (tid < EPI_T1) {
-    const int u = tid & 3, slot = (tid >> 2) & 7, pt = (tid >> 5) / 3, ht = (tid >> 5) % 3;
+  for (int x = wave * 64 + lane; x < EPI_T1; x += 64 * NW) {
+    const int u = x & 3, slot = (x >> 2) & 7, pt = (x >> 5) / 3, ht = (x >> 5) % 3;
     const int p = pt == 0 ? particle(G.a, slot)
                           : (pt == 1 ? particle(G.b, slot) : particle(G.c, slot));
     const int h = ht == 0 ? hole(G.I, u) : (ht == 1 ? hole(G.J, u) : hole(G.K, u));
-    e[EPI_S + tid] = T1[p * no + h];
+    e[EPI_S + x] = T1[p * ldp + h * ldh];
   }
+}
+// The singles operands of a job.
+template <int NW>
+__device__ __forceinline__ void stage_singles(double *e, cptr<FusedArgs> A, int wave, int lane,
+                                              const ItemGeo &G) {
+  stage_epilogue<NW>(e, (gptr<const double>)A->S, A->nv, (gptr<const double>)A->T1, A->no, 1, A->no,
+                     A->nv, wave, lane, G);
 }
 
 // A lane's place in its item: particle slots in the box (sa, sb, sc), local
@@ -806,6 +855,10 @@ __device__ __forceinline__ Denominator denominator(cptr<FusedArgs> A, const Item
   return D;
 }
 
+// Between the parts of an epilogue: no instruction moves across, so that the
+// arrays of one part are dead before those of the next are live.
+__device__ __forceinline__ void phase() { __builtin_amdgcn_sched_barrier(0); }
+
 // v[r] = f(i, j, k, r), r = 16 i + 4 j + k, over the lane's elements, 0 in the
 // hole pairs (j, k) past a ragged edge.
 template <class F>
@@ -823,23 +876,44 @@ __device__ __forceinline__ void each_element(const ItemGeo &G, double (&v)[64], 
     }
 }
 
+// The same with the element's value x in the spill slot: v[r] = f(i, j, k, x),
+// read 16 at a time (one wait each, not one per hole pair).
+template <class F>
+__device__ __forceinline__ void each_element_with(const ItemGeo &G, gptr<const double> in, int lane,
+                                                  double (&v)[64], F &&f) {
+#pragma unroll
+  for (int jj = 0; jj < 4; ++jj) {
+    double x[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+      v[16 * (n >> 2) + 4 * jj + (n & 3)] = 0.0;
+      x[n] = in[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
+    }
+    if (jj < G.J.n)
+#pragma unroll
+      for (int n = 0; n < 16; ++n)
+        if ((n & 3) < G.K.n) v[16 * (n >> 2) + 4 * jj + (n & 3)] = f(n >> 2, jj, n & 3, x[n]);
+    phase();
+  }
+}
+
 // f(r, factor of the singles product of element r) over the 9 singles
 // products of the lane's elements, r = 16 i + 4 j + k, from the staged
 // operands; the elements of one hole pair past a ragged edge are skipped.
 template <class F>
 __device__ __forceinline__ void each_single(const double *e, const ItemGeo &G, const Place &p,
                                             F &&f) {
-  const int obc = 0 * 64 + p.sb * 8 + p.sc, oac = 1 * 64 + p.sa * 8 + p.sc,
-            oab = 2 * 64 + p.sa * 8 + p.sb;
+  const int sa = again(p.sa), sb = again(p.sb), sc = again(p.sc);
+  const int obc = 0 * 64 + sb * 8 + sc, oac = 1 * 64 + sa * 8 + sc, oab = 2 * 64 + sa * 8 + sb;
   const double *t1 = e + EPI_S;
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
     double ta[4], tb[4], tc[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      ta[u] = t1[((0 * 3 + t) * 8 + p.sa) * 4 + u];
-      tb[u] = t1[((1 * 3 + t) * 8 + p.sb) * 4 + u];
-      tc[u] = t1[((2 * 3 + t) * 8 + p.sc) * 4 + u];
+      ta[u] = t1[((0 * 3 + t) * 8 + sa) * 4 + u];
+      tb[u] = t1[((1 * 3 + t) * 8 + sb) * 4 + u];
+      tc[u] = t1[((2 * 3 + t) * 8 + sc) * 4 + u];
     }
     const double sg = t == 1 ? -1.0 : 1.0;
     const int n1 = t == 0 ? G.J.n : G.I.n, n2 = t == 2 ? G.J.n : G.K.n;
@@ -937,58 +1011,18 @@ constexpr bool pair_epilogue(int epi) { return epi == EPI_LAMBDA || epi == EPI_C
 // and two passes over it in HBM.
 
 // Left-hand half of a Lambda item: the y3 doubles, i.e. the accumulators plus
-// the Fock term P(c/ab) P(k/ij) y(a b i j) f(k c), y from the job's dense T2e
-// (T2e[i][j][a][b] = y(a b i j)).  Elements outside the task are written too
-// (the right-hand half skips them).
+// the Fock term P(c/ab) P(k/ij) y(a b i j) f(k c).  Written out, that term is
+// the singles term with f(h p) for t1(p h) and y(p p' h h') for S: its operands
+// are staged and summed as those (`fock`; y from the job's dense T2e, T2e[h][h'][p][p']).
+// Elements outside the task are written too (the right-hand half skips them).
 template <class Q>
-__device__ __forceinline__ void lambda_left(const Q (&q)[16], cptr<MixedArgs> M, cptr<TaskDev> T,
+__device__ __forceinline__ void lambda_left(const Q (&q)[16], const double *e, bool fock,
                                             const Place &p, const ItemGeo &G, gptr<double> out,
                                             int lane) {
-  const cptr<FusedArgs> A = &M->f;
   double yd[64];
 #pragma unroll
   for (int r = 0; r < 64; ++r) yd[r] = (double)q[r & 15][r >> 4];
-  if (M->lam_f && inside(T, p)) {
-    const int no = A->no, nv = A->nv;
-    const long Ep = A->Ep;
-    const int a = particle(G.a, p.sa), b = particle(G.b, p.sb), c = particle(G.c, p.sc);
-    const gptr<const double> Y = (gptr<const double>)A->T2e, F = (gptr<const double>)M->lam_f;
-    auto y = [&](int u, int v, int h, int g) { return Y[(((long)h * no + g) * nv + u) * Ep + v]; };
-    // g(h1, h2, h3) = y(a b h1 h2) f(h3 c) - y(c b h1 h2) f(h3 a) - y(a c h1 h2) f(h3 b);
-    // the term is g(i, j, k) - g(k, j, i) - g(i, k, j).  T = 0: g(i, j, k);
-    // T = 1: -g(k, j, i); T = 2: -g(i, k, j).  Outer loops over (h1, h2),
-    // inner over h3, whose three f values are loaded once per term; hole
-    // pairs past a ragged edge are skipped.
-#pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      const HoleBox H1 = t == 1 ? G.K : G.I, H2 = t == 2 ? G.K : G.J,
-                    H3 = t == 0 ? G.K : (t == 1 ? G.I : G.J);
-      const double sg = t == 0 ? 1.0 : -1.0;
-      double fc[4], fa[4], fb[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const long h3 = (long)hole(H3, u) * nv;
-        fc[u] = F[h3 + c];
-        fa[u] = F[h3 + a];
-        fb[u] = F[h3 + b];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          if (!(u < H1.n && w < H2.n)) continue;
-          const int h1 = hole(H1, u), h2 = hole(H2, w);
-          const double yab = sg * y(a, b, h1, h2), ycb = sg * y(c, b, h1, h2),
-                       yac = sg * y(a, c, h1, h2);
-#pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            // (h1, h2, h3) = (u, w, m) in the order of (i, j, k) for the term
-            const int ii = t == 1 ? m : u, jj = t == 2 ? m : w, kk = t == 0 ? m : (t == 1 ? u : w);
-            yd[16 * ii + 4 * jj + kk] += yab * fc[m] - ycb * fa[m] - yac * fb[m];
-          }
-        }
-    }
-  }
+  if (fock) each_single(e, G, p, [&](int r, double s) { yd[r] += s; });
 #pragma unroll
   for (int r = 0; r < 64; ++r) out[r * 64 + lane] = yd[r];
 }
@@ -999,6 +1033,7 @@ __device__ __forceinline__ void cr_left(const Q (&q)[16], const double *e, const
                                         const ItemGeo &G, gptr<double> out, int lane) {
 #pragma unroll
   for (int r = 0; r < 64; ++r) out[r * 64 + lane] = (double)q[r & 15][r >> 4];
+  phase();
   double sv[64];
   singles_products(e, G, p, sv);
 #pragma unroll
@@ -1020,13 +1055,14 @@ __device__ __forceinline__ void lambda_right(const Q (&q)[16], const double *e, 
   const Denominator D = denominator(A, G, p);
   const double factor = T->factor;
   double den[64];
-  each_element(G, den, [&](int ii, int jj, int kk, int r) {
+  each_element_with(G, in, lane, den, [&](int ii, int jj, int kk, double yd) {
     const double dn = (double)q[4 * jj + kk][ii] * factor /
                       (D.eh[0][ii] + D.eh[1][jj] + D.eh[2][kk] + D.d0);
     const bool ok = ii < G.I.n;
-    e1 += ok ? dn * in[r * 64 + lane] : 0.0;
+    e1 += ok ? dn * yd : 0.0;
     return ok ? dn : 0.0;
   });
+  phase();
   double x = 0.0;
   each_single(e, G, p, [&](int r, double s) { x += den[r] * s; });
   e2 = e1 + x;
@@ -1045,44 +1081,66 @@ __device__ __forceinline__ void cr_right(const Q (&q)[16], const double *e, cptr
   if (!inside(T, p)) return;
   const Denominator D = denominator(A, G, p);
   const double factor = T->factor;
-  // the singles q_r enter sum-wise: s2 = sum (w td)_r q_r, s3 = s2 + sum (w
-  // ts)_r q_r, one 64-value array live at a time
+  double d0 = D.d0;
   auto weight = [&](int ii, int jj, int kk) {
-    const double w = factor / (D.eh[0][ii] + D.eh[1][jj] + D.eh[2][kk] + D.d0);
+    const double w = factor / (D.eh[0][ii] + D.eh[1][jj] + D.eh[2][kk] + d0);
     return ii < G.I.n ? w : 0.0;
   };
-  double v[64];
-  each_element(G, v, [&](int ii, int jj, int kk, int r) {
-    const double w = weight(ii, jj, kk), rd = (double)q[4 * jj + kk][ii] * w;
-    const double td = in[r * 64 + lane], ts = in[(64 + r) * 64 + lane];
-    s[0] += rd * td;
-    s[1] += rd * (td + ts);
-    return w * td;
-  });
-  each_single(e, G, p, [&](int r, double x) { s[2] += v[r] * x; });
-  each_element(G, v, [&](int ii, int jj, int kk, int r) {
-    return weight(ii, jj, kk) * in[(64 + r) * 64 + lane];
-  });
-  s[3] = s[2];
-  each_single(e, G, p, [&](int r, double x) { s[3] += v[r] * x; });
+  // the accumulators are read out first, then one 64-value array is live at a
+  // time (both together do not fit the registers; a third division is cheaper)
+  const gptr<const double> ins = in + 64 * 64;
+#pragma unroll
+  for (int jj = 0; jj < 4; ++jj) {
+    double td[16], ts[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+      td[n] = in[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
+      ts[n] = ins[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
+    }
+    if (jj < G.J.n)
+#pragma unroll
+      for (int n = 0; n < 16; ++n)
+        if ((n & 3) < G.K.n) {
+          const double rd = (double)q[4 * jj + (n & 3)][n >> 2] * weight(n >> 2, jj, n & 3);
+          s[0] += rd * td[n];
+          s[1] += rd * ts[n];
+        }
+  }
+  s[1] += s[0];
+  phase();
+#pragma unroll 1
+  for (int half = 0; half < 2; ++half) {
+    double v[64];
+    asm volatile("" : "+v"(d0));  // the 64 weights anew, not kept from the loop above
+    each_element_with(G, half ? ins : in, lane, v, [&](int ii, int jj, int kk, double t) {
+      return weight(ii, jj, kk) * t;
+    });
+    phase();
+    each_single(e, G, p, [&](int r, double x) { s[3] += v[r] * x; });
+    if (!half) s[2] = s[3];
+  }
 }
 
 // The item loop, with the epilogue EPI.
 template <int PREC, int EPI>
-__global__ void __launch_bounds__(512) fused_triples_mixed(const MixedSegment *segments, int nseg,
+__global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(const MixedSegment *segments, int nseg,
                                                            long nglobal,
                                                            unsigned long long *sched) {
   __shared__ f4 lds[lds_quads<PREC>()];
   __shared__ long next_item;  // dynamic schedule: the workgroup's next item
   using Pr = Prec<PREC>;
+  constexpr int NW = Pr::NW;
+  constexpr bool HALF = NW == 4;  // the launch's indices are half items
+  if (HALF) nglobal *= 2;
   const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = tid & 63;
-  const unsigned lds_base = (unsigned)(unsigned long)(__attribute__((address_space(3))) f4 *)lds;
+  const unsigned lds_base =
+      (unsigned)uniform((int)(unsigned long)(__attribute__((address_space(3))) f4 *)lds);
   const cptr<MixedSegment> segs = (cptr<MixedSegment>)segments;
   // Persistent loop over the launch's items, uniform across the workgroup
   // (every barrier is reached by all 8 waves): the dynamic schedule of
   // sched_item when `sched` is given, else a static round-robin.
   const bool dyn = sched != nullptr;
-  const int sh = dyn ? (int)sched[9] : 0;  // log2 of the slice width
+  const int sh = (dyn ? (int)sched[9] : 0) + (HALF ? 1 : 0);  // log2 of the slice width
   unsigned queue = blockIdx.x & 7u;  // thread 0: the queue it draws from
   unsigned long long ticket = 0;
   long g = 0;
@@ -1102,8 +1160,10 @@ __global__ void __launch_bounds__(512) fused_triples_mixed(const MixedSegment *s
       g = round_item(r, blockIdx.x, gridDim.x, nseg > 1);
       if (g >= nglobal) continue;  // last round: uniform per workgroup
     }
-    seg = next_segment(segs, nseg, seg, g);
-    const long item = segs[seg].item0 + (g - segs[seg].g0);
+    const long gi = HALF ? g >> 1 : g;
+    const int c4 = HALF ? 4 * (int)(g & 1) : 0;  // first c slot of a half item
+    seg = next_segment(segs, nseg, seg, gi);
+    const long item = segs[seg].item0 + (gi - segs[seg].g0);
     const cptr<MixedArgs> M = (cptr<MixedArgs>)segs[seg].args;
     const cptr<FusedArgs> A = &M->f;
     const cptr<TaskDev> tasks = (cptr<TaskDev>)A->tasks;
@@ -1123,21 +1183,28 @@ __global__ void __launch_bounds__(512) fused_triples_mixed(const MixedSegment *s
     G.I = hbox(T->oh1, bi, T->r1);
     G.J = hbox(T->oh2, bj, T->r2);
     G.K = hbox(T->oh3, bk, T->r3);
-    auto prng = [](int o, int b, int r) { return PRange{o + 8 * b, min(7, r - 1 - 8 * b), 0}; };
-    G.a = prng(T->op4, ba, T->r4);
-    G.b = prng(T->op5, bb, T->r5);
-    G.c = prng(T->op6, bc, T->r6);
+    auto prng = [](int o, int r, int n) { return PRange{o, min(n - 1, r - 1), 0}; };
+    G.a = prng(T->op4 + 8 * ba, T->r4 - 8 * ba, 8);
+    G.b = prng(T->op5 + 8 * bb, T->r5 - 8 * bb, 8);
+    G.c = prng(T->op6 + 8 * bc + c4, T->r6 - 8 * bc - c4, HALF ? 4 : 8);
     {
       // wave bits of the cube coordinates: the ranges with two cubes take the
       // low bits, so the waves with work spread over the four SIMDs (wave w
       // runs on SIMD w % 4)
       const bool wa = G.a.sm >= 4, wb = G.b.sm >= 4, wc = G.c.sm >= 4;
-      const int nw = (wa ? 1 : 0) + (wb ? 1 : 0) + (wc ? 1 : 0);
-      G.c.bit = wc ? 0 : nw;
-      G.b.bit = wb ? (wc ? 1 : 0) : nw + (wc ? 0 : 1);
-      G.a.bit = wa ? (wc ? 1 : 0) + (wb ? 1 : 0) : nw + (wc ? 0 : 1) + (wb ? 0 : 1);
+      if (HALF) {
+        G.b.bit = wb || !wa ? 0 : 1;
+        G.a.bit = 1 - G.b.bit;
+        G.c.bit = 2;  // one cube
+      } else {
+        const int nw = (wa ? 1 : 0) + (wb ? 1 : 0) + (wc ? 1 : 0);
+        G.c.bit = wc ? 0 : nw;
+        G.b.bit = wb ? (wc ? 1 : 0) : nw + (wc ? 0 : 1);
+        G.a.bit = wa ? (wc ? 1 : 0) + (wb ? 1 : 0) : nw + (wc ? 0 : 1) + (wb ? 0 : 1);
+      }
     }
-    const ItemPlan P = item_plan(T->eq);
+    const ItemPlan P = item_plan(T->eq, HALF);
+    const long part = item * 8 + c4 + wave;  // the wave's partial
 
     double *epi = reinterpret_cast<double *>(lds);
     Place p;  // layout c: lane = 4a' + b' + 16c'
@@ -1146,23 +1213,33 @@ __global__ void __launch_bounds__(512) fused_triples_mixed(const MixedSegment *s
       p.sa = 4 * cube(wave, G.a) + ((ln & 15) >> 2);
       p.sb = 4 * cube(wave, G.b) + (ln & 3);
       p.sc = 4 * cube(wave, G.c) + (ln >> 4);
-      p.la = 8 * ba + p.sa, p.lb = 8 * bb + p.sb, p.lc = 8 * bc + p.sc;
+      p.la = 8 * ba + p.sa, p.lb = 8 * bb + p.sb, p.lc = 8 * bc + c4 + p.sc;
       p.i0 = 4 * bi, p.j0 = 4 * bj, p.k0 = 4 * bk;
     }
     const gptr<double> partials = (gptr<double>)A->partials;
+    const gptr<double> den = (gptr<double>)M->cr_den;
+    const bool empty = HALF && G.c.sm < 0;  // a half past the edge: no element
+    if (empty && EPI != EPI_TILES && lane == 0) {
+      partials[2 * part] = partials[2 * part + 1] = 0.0;
+      if (EPI == EPI_CR) den[2 * part] = den[2 * part + 1] = 0.0;
+    }
     // one half, or the left-hand and the right-hand half of a pair's item (the
     // jobs have the same tasks)
 #pragma unroll 1
-    for (int side = pair_epilogue(EPI) ? 0 : 1; side < 2; ++side) {
+    for (int side = empty ? 2 : (pair_epilogue(EPI) ? 0 : 1); side < 2; ++side) {
       const cptr<MixedArgs> ML = (cptr<MixedArgs>)M->left;
       const cptr<MixedArgs> MS = side ? M : ML;
       typename Pr::quad q[16];
       contract<PREC>(q, lds, lds_base, MS, T, G, P, wave, lane);
       // Epilogue: the chunk buffers are free.
-      const long slot = ((long)blockIdx.x * 8 + wave) * (EPI == EPI_CR ? 8192 : 4096);
+      const long slot = ((long)blockIdx.x * NW + wave) * (EPI == EPI_CR ? 8192 : 4096);
       const gptr<double> spill = (gptr<double>)M->spill + slot;
-      if (EPI != EPI_LAMBDA || side)
-        stage_epilogue(epi, EPI == EPI_LAMBDA ? &ML->f : &MS->f, wave, lane, G);
+      const bool fock = EPI == EPI_LAMBDA && side == 0 && ML->lam_f != nullptr;
+      if (fock)
+        stage_epilogue<NW>(epi, (gptr<const double>)ML->f.T2e, ML->f.Ep,
+                           (gptr<const double>)ML->lam_f, 1, A->nv, A->no, A->nv, wave, lane, G);
+      else if (EPI != EPI_LAMBDA || side)
+        stage_singles<NW>(epi, EPI == EPI_LAMBDA ? &ML->f : &MS->f, wave, lane, G);
       __syncthreads();
       if constexpr (EPI == EPI_TILES) {
         store_tiles(q, epi, A, T, p, G);
@@ -1171,32 +1248,31 @@ __global__ void __launch_bounds__(512) fused_triples_mixed(const MixedSegment *s
         energy(q, epi, A, T, p, G, e4, e5);
         wave_sum(e4, e5);
         if (lane == 0) {
-          partials[2 * (item * 8 + wave)] = e4;
-          partials[2 * (item * 8 + wave) + 1] = e5;
+          partials[2 * part] = e4;
+          partials[2 * part + 1] = e5;
         }
       } else if (side == 0) {
-        if constexpr (EPI == EPI_LAMBDA) lambda_left(q, ML, T, p, G, spill, lane);
-        else cr_left(q, epi, p, G, spill, lane);
+        if constexpr (EPI == EPI_LAMBDA) lambda_left(q, epi, fock, p, G, spill, again(lane));
+        else cr_left(q, epi, p, G, spill, again(lane));
         __syncthreads();  // the right-hand half's first loads overwrite the staged data
       } else if constexpr (EPI == EPI_LAMBDA) {
         double e1, e2;
-        lambda_right(q, epi, A, T, p, G, spill, lane, e1, e2);
+        lambda_right(q, epi, A, T, p, G, spill, again(lane), e1, e2);
         wave_sum(e1, e2);
         if (lane == 0) {
-          partials[2 * (item * 8 + wave)] = e1;
-          partials[2 * (item * 8 + wave) + 1] = e2;
+          partials[2 * part] = e1;
+          partials[2 * part + 1] = e2;
         }
       } else {
         double cs[4];
-        cr_right(q, epi, A, T, p, G, spill, lane, cs);
+        cr_right(q, epi, A, T, p, G, spill, again(lane), cs);
         wave_sum(cs[0], cs[1]);
         wave_sum(cs[2], cs[3]);
         if (lane == 0) {
-          const gptr<double> den = (gptr<double>)M->cr_den;
-          partials[2 * (item * 8 + wave)] = cs[0];
-          partials[2 * (item * 8 + wave) + 1] = cs[1];
-          den[2 * (item * 8 + wave)] = cs[2];
-          den[2 * (item * 8 + wave) + 1] = cs[3];
+          partials[2 * part] = cs[0];
+          partials[2 * part + 1] = cs[1];
+          den[2 * part] = cs[2];
+          den[2 * part + 1] = cs[3];
         }
       }
     }
@@ -1209,14 +1285,16 @@ __global__ void __launch_bounds__(512) fused_triples_mixed(const MixedSegment *s
 
 }  // namespace
 
-// The contraction extents of every job in the table must be multiples of
+// grid: workgroups of 8 waves, at most one per CU (halves: twice as many of 4
+// waves).  The contraction extents of every job in the table must be multiples of
 // the precision's chunk (8 FP64 / 16 FP32 / 32 bf16 values); the job layer
 // pads them.
 template <int PREC, int EPI>
 static void launch_one(const MixedSegment *segs, int nseg, long total, int grid, hipStream_t s,
                        unsigned long long *sched) {
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(fused_triples_mixed<PREC, EPI>), dim3((unsigned)grid),
-                     dim3(512), 0, s, segs, nseg, total, sched);
+  constexpr int NW = Prec<PREC>::NW;
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(fused_triples_mixed<PREC, EPI>), dim3((unsigned)grid * 8 / NW),
+                     dim3(64 * NW), 0, s, segs, nseg, total, sched);
 }
 template <int EPI>
 static int launch_prec(const MixedSegment *segs, int nseg, long total, int precision, int grid,

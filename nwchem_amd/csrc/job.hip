@@ -234,11 +234,10 @@ struct ClassRanges {
       const int sp = q.kind == 1 ? 0 : 1;
       const bool ok = spin >= 0 && spin <= 3 && sym >= 0 && sym <= 7;
       if (whole) {
-        d.x0[p] = 0, d.x1[p] = (unsigned short)(sp ? T.nv : T.no);
+        d.x[p] = (unsigned)(sp ? T.nv : T.no) << 16;
         continue;
       }
-      d.x0[p] = ok ? (unsigned short)lo[sp][spin][sym] : 0;
-      d.x1[p] = ok ? (unsigned short)hi[sp][spin][sym] : 0;
+      d.x[p] = ok ? (unsigned)lo[sp][spin][sym] | (unsigned)hi[sp][spin][sym] << 16 : 0;
     }
   }
 };
@@ -288,6 +287,11 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
     int kp[3], kh[3];
     order3(p, kp);
     order3(h, kh);
+    // a pair of equal particle boxes goes first (fused_triples_mixed splits c)
+    if (p[kp[1]].o == p[kp[2]].o && p[kp[0]].o != p[kp[1]].o) {
+      const int k0 = kp[0];
+      kp[0] = kp[1], kp[1] = kp[2], kp[2] = k0;
+    }
     d.op4 = p[kp[0]].o, d.op5 = p[kp[1]].o, d.op6 = p[kp[2]].o;
     d.oh1 = h[kh[0]].o, d.oh2 = h[kh[1]].o, d.oh3 = h[kh[2]].o;
     d.r4 = p[kp[0]].r, d.r5 = p[kp[1]].r, d.r6 = p[kp[2]].r;
@@ -301,8 +305,7 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
       cr.set(T, t, r.d);
       r.set = true;
     }
-    std::copy(r.d.x0, r.d.x0 + 18, d.x0);
-    std::copy(r.d.x1, r.d.x1 + 18, d.x1);
+    std::copy(r.d.x, r.d.x + 18, d.x);
   };
   // sub-tiles of tile b with edge e (the last one ragged)
   auto pieces = [&](long b, int e, bool hole) {
