@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -165,11 +166,17 @@ struct CallArgs {
 // element of the hole block at TA x TB places of the particle indices, TA of
 // one that sits on the a operand and TB of one that sits on b: TA + TB operand
 // loads feed TA TB multiply-adds, and lanes read and write consecutive
-// elements of t3.
+// elements of t3.  The d1/d2 operands are packed first (pack_operands): the
+// hole indices fastest, in the output's order, then the contraction index, so
+// that lanes read consecutive operand elements too (t2sub and the d2 v2sub
+// have the contraction index fastest: every lane on a line of its own).
 // Bound: HBM, 16 bytes per element of t3 (read and written on each call; the
 // operands stay in L2), at tiles of 12^3 x 24^3 elements 82 us at the 4.7 TB/s
-// of a plain copy.  One element per thread, with two loads per multiply-add
-// and six 64-bit divisions per element, took 584 us per call on average.
+// of a plain copy.  Time per call there: one element per thread, with two
+// loads per multiply-add and six 64-bit divisions per element, 584 us on
+// average; 4 x 4 tiles on the operands as they come s1 74, d1 117 to 208, d2
+// 215 to 528 us; packed (4 to 10 us
+// more) s1 74, d1 114, d2 164 us.
 constexpr int TA = 4, TB = 4;
 struct DirectArgs {
   unsigned F, d0, d1;          // hole block, its two fastest extents
@@ -185,6 +192,64 @@ struct DirectArgs {
   double sign;
 };
 
+// Whether operand a (t1sub / t2sub) of a family has the index.
+bool on_a(int family, int code) {
+  return code == P4 || code == H1 || (family == 1 && code == P5) || (family == 2 && code == H2);
+}
+
+// A packed copy of one operand: dims in the packed order (holes in the
+// output's order, contraction index, particles), source strides.
+struct PackArgs {
+  unsigned n;
+  unsigned ext[5];
+  long src[5];
+};
+struct PackPair {
+  PackArgs p[2];  // a, b
+  long at[2];     // source offsets (elements)
+  long to[2];     // packed offsets
+};
+
+__global__ void __launch_bounds__(256) pack_operands(PackPair P, const double *__restrict__ in,
+                                                     double *__restrict__ out) {
+  const PackArgs &p = P.p[blockIdx.y];
+  const unsigned x = blockIdx.x * 256u + threadIdx.x;
+  if (x >= p.n) return;
+  unsigned r = x;
+  long o = 0;
+#pragma unroll
+  for (int q = 0; q < 5; ++q) {
+    const unsigned v = r % p.ext[q];
+    r /= p.ext[q];
+    o += v * p.src[q];
+  }
+  out[P.to[blockIdx.y] + x] = in[P.at[blockIdx.y] + o];
+}
+
+// The packed form of a call's operand (a or b): fills p and replaces the
+// operand's strides in c.
+PackArgs pack_args(CallArgs &c, int family, bool a) {
+  PackArgs p;
+  long *st = a ? c.sa : c.sb;
+  long &ks = a ? c.ka : c.kb;
+  int q = 0;
+  long at = 1;
+  auto dim = [&](long ext, long &stride) {
+    p.ext[q] = (unsigned)ext;
+    p.src[q++] = stride;
+    stride = at;
+    at *= ext;
+  };
+  for (int k = 0; k < 3; ++k)
+    if (on_a(family, c.codeL[k]) == a) dim(c.dimL[k], st[c.codeL[k]]);
+  dim(c.K, ks);
+  for (int k = 3; k < 6; ++k)
+    if (on_a(family, c.codeL[k]) == a) dim(c.dimL[k], st[c.codeL[k]]);
+  p.n = (unsigned)at;
+  for (; q < 5; ++q) p.ext[q] = 1, p.src[q] = 0;
+  return p;
+}
+
 DirectArgs direct_args(const CallArgs &c, int family) {
   DirectArgs d;
   long stride[6], s = 1;
@@ -194,9 +259,9 @@ DirectArgs direct_args(const CallArgs &c, int family) {
   for (int q = 0; q < 3; ++q) d.fa[q] = c.sa[c.codeL[q]], d.fb[q] = c.sb[c.codeL[q]];
   int qa = -1, qb = -1, qc = -1;
   for (int q = 3; q < 6; ++q) {
-    const bool on_a = c.codeL[q] == P4 || (family == 1 && c.codeL[q] == P5);
-    if (on_a && qa < 0) qa = q;
-    else if (!on_a && qb < 0) qb = q;
+    const bool a = on_a(family, c.codeL[q]);
+    if (a && qa < 0) qa = q;
+    else if (!a && qb < 0) qb = q;
     else qc = q;
   }
   d.na = (int)c.dimL[qa], d.nb = (int)c.dimL[qb];
@@ -240,7 +305,7 @@ __global__ void __launch_bounds__(256) contract_kernel(DirectArgs c, double *__r
       acc[u][v] = 0.0;
       old[u][v] = pa + u < c.na && pb + v < c.nb ? t[u * c.a_t + v * c.b_t] : 0.0;
     }
-#pragma unroll 2
+#pragma unroll 4
   for (int k = 0; k < c.K; ++k) {
     double av[TA], bv[TB];
 #pragma unroll
@@ -359,7 +424,9 @@ void launch_call(int family, int n, const long dims[6], long K, const double *ha
   }
   memcpy(S.pinned, ha, na * sizeof(double));
   memcpy(S.pinned + na, hb, nb * sizeof(double));
-  double *dops = (double *)S.pool.get(bytes);
+  // the direct d1/d2 contractions read packed copies behind the operands
+  const bool pack = family != 0 && backend_of(S) == TCE_T_LEGACY_DIRECT && K > 0;
+  double *dops = (double *)S.pool.get(pack ? 2 * bytes : bytes);
   if (!dops) {
     set_error("device pool allocation failed");
     S.failed = true;
@@ -421,9 +488,22 @@ void launch_call(int family, int n, const long dims[6], long K, const double *ha
                        t3, dC);
     if (!ok(hipGetLastError(), "permute_add_kernel launch")) return;
   } else {
+    const double *ops = dops;
+    if (pack) {
+      PackPair P;
+      P.p[0] = pack_args(c, family, true);
+      P.p[1] = pack_args(c, family, false);
+      P.at[0] = P.to[0] = 0;
+      P.at[1] = P.to[1] = na;
+      double *packed = dops + na + nb;
+      hipLaunchKernelGGL(pack_operands, dim3((std::max(P.p[0].n, P.p[1].n) + 255) / 256, 2),
+                         dim3(256), 0, S.stream, P, dops, packed);
+      if (!ok(hipGetLastError(), "pack_operands launch")) return;
+      ops = packed;
+    }
     const DirectArgs da = direct_args(c, family);
     hipLaunchKernelGGL(contract_kernel, dim3((da.threads + 255) / 256, da.nc), dim3(256), 0,
-                       S.stream, da, t3, dops, dops + na);
+                       S.stream, da, t3, ops, ops + na);
     if (!ok(hipGetLastError(), "contract_kernel launch")) return;
   }
   if (host_t3 && !ok(hipMemcpyAsync(host_t3, t3, tbytes, hipMemcpyDeviceToHost, S.stream), "D2H t3"))
