@@ -66,10 +66,10 @@
 // unrolled it was 84 KB, more than the 64 KB instruction cache two CUs share,
 // and every item ran from L2.
 //
-// Together (one box, ms before / after): no=40/nv=160 FP64 635 / 521, no=21/
-// nv=160 in ragged tiles 149 / 92, no=26/nv=114 in spin-labelled ragged tiles
-// 17.7 / 7.5, no=40/nv=320 in 2 spins x 4 irreps (tiles of 5 holes) 446 / 209,
-// bf16x6 no=40/nv=200 526 / 477.
+// Together (ms before / after): no=40/nv=160 FP64 635 / 472, no=21/nv=160 in
+// ragged tiles 149 / 81, no=26/nv=114 in spin-labelled ragged tiles 17.7 /
+// 5.8, no=40/nv=320 in 2 spins x 4 irreps (tiles of 5 holes) 446 / 189,
+// bf16x6 no=40/nv=200 526 / 456.
 //
 // LDS layout of one buffer part (hi or lo; quads, kq = quad 0..3 of a row):
 //   X  [4 s][8 L slots][4 r][4 kq ^ x_swz]         512 quads
@@ -552,21 +552,29 @@ __device__ __forceinline__ void chunk_loop(typename Prec<PREC>::quad (&q)[16], c
     const int nb = st.buf + AH < NB ? st.buf + AH : st.buf + AH - NB;
     const unsigned nbase = lds_base + (unsigned)nb * (buf_quads<PREC>() * 16u);
     const bool more = st.todo > 0;
-    // the MFMAs of X quad s
+    // the MFMAs of X quad s with Y quads 0..h1-1; all four term by term, so that
+    // dependent MFMAs on one quad are 4 instructions apart
+    auto quad = [&](int s, int h) {
+#pragma unroll
+      for (int t = 0; t < terms<PREC>(); ++t)
+        q[qi<KP>(s, h)] = mma<PREC>(f, s, h, t, q[qi<KP>(s, h)]);
+    };
+    // The masks are nested, so that a short row leaves at its first absent quad
+    // and a full one takes one branch: tested quad by quad, the 16 tests of a
+    // chunk made no=40/nv=160 484 ms instead of 472, and 201 instead of 189 in
+    // tiles of 5 holes (no=40/nv=320 in irreps, one quad to a row in most items).
     auto row = [&](int s) {
-      if (s < s0 || s >= s1) return;
       if (h1 == 4) {
 #pragma unroll
         for (int t = 0; t < terms<PREC>(); ++t)
 #pragma unroll
           for (int h = 0; h < 4; ++h) q[qi<KP>(s, h)] = mma<PREC>(f, s, h, t, q[qi<KP>(s, h)]);
       } else {
-#pragma unroll
-        for (int h = 0; h < 3; ++h)
-          if (h < h1)
-#pragma unroll
-            for (int t = 0; t < terms<PREC>(); ++t)
-              q[qi<KP>(s, h)] = mma<PREC>(f, s, h, t, q[qi<KP>(s, h)]);
+        quad(s, 0);
+        if (h1 > 1) {
+          quad(s, 1);
+          if (h1 > 2) quad(s, 2);
+        }
       }
     };
     if (s1 > 0) {
@@ -574,16 +582,16 @@ __device__ __forceinline__ void chunk_loop(typename Prec<PREC>::quad (&q)[16], c
       for (int h = 0; h < 4; ++h) read_y<PREC>(f, cb, o.y, h);
 #pragma unroll
       for (int s = 0; s < 4; ++s) read_x<PREC>(f, cb, o.x, s);
-      row(0);
-      row(1);
+      if (s0 == 0) row(0);
+      if (s1 > 1) row(1);
     }
     if (NB >= 3 && more) {
       nl = st.ld.load(A, T, G, P, nbase, wave, lane);
       --st.todo;
     }
-    if (s1 > 0) {
+    if (s1 > 2) {
       row(2);
-      row(3);
+      if (s1 > 3) row(3);
     }
     // chunk j+1 landed once at most the loads of the later ones are pending
     if constexpr (NB == 3) wait_vm_n(nl);
