@@ -66,9 +66,9 @@
 // unrolled it was 84 KB, more than the 64 KB instruction cache two CUs share,
 // and every item ran from L2.
 //
-// Together (ms before / after): no=40/nv=160 FP64 635 / 472, no=21/nv=160 in
-// ragged tiles 149 / 81, no=26/nv=114 in spin-labelled ragged tiles 17.7 /
-// 5.8, no=40/nv=320 in 2 spins x 4 irreps (tiles of 5 holes) 446 / 189,
+// Together (ms before / after): no=40/nv=160 FP64 635 / 462, no=21/nv=160 in
+// ragged tiles 149 / 79, no=26/nv=114 in spin-labelled ragged tiles 17.7 /
+// 5.7, no=40/nv=320 in 2 spins x 4 irreps (tiles of 5 holes) 446 / 185,
 // bf16x6 no=40/nv=200 526 / 456.
 //
 // LDS layout of one buffer part (hi or lo; quads, kq = quad 0..3 of a row):
@@ -191,6 +191,20 @@ __device__ __forceinline__ int particle(const PRange &p, int slot) { return p.g0
 struct ItemGeo {
   HoleBox I, J, K;
   PRange a, b, c;
+  int heq;  // EQ_IJ, EQ_JK of a one-box task
+  // Whether the pair (u, w) of hole boxes t (0: (j,k), 1: (i,k), 2: (i,j)) has
+  // elements that count: inside the boxes, and u < w when the two are one box
+  // (the rest follow by antisymmetry, distinct() of them alike).  The epilogue
+  // of an item with I == J == K forms 4 elements of a particle triple, not 64:
+  // no=8/nv=32 153 us before, 134 after; no=40/nv=160 472 and 462 ms.
+  __device__ __forceinline__ bool pair(int t, int u, int w) const {
+    const int n1 = t == 0 ? J.n : I.n, n2 = t == 2 ? J.n : K.n;
+    const int m = t == 0 ? EQ_JK : (t == 2 ? EQ_IJ : EQ_IJ | EQ_JK);
+    return u < n1 && w < n2 && !((heq & m) == m && u >= w);
+  }
+  __device__ __forceinline__ double distinct() const {
+    return heq == 0 ? 1.0 : (heq == (EQ_IJ | EQ_JK) ? 6.0 : 2.0);
+  }
 };
 // Chosen field by field: a choice between the structs themselves would put G
 // in scratch memory.
@@ -812,7 +826,7 @@ __device__ __forceinline__ void stage_epilogue(double *e, gptr<const double> S, 
       const int tp = wave + NW * r, t = (NW * r) >> 4, u = (tp >> 2) & 3, w = tp & 3;
       const HoleBox H1 = hole_box(G, t == 0 ? 1 : 0), H2 = hole_box(G, t == 2 ? 1 : 2);
       v[r] = 0.0;
-      if (u < H1.n && w < H2.n)
+      if (G.pair(t, u, w))
         v[r] = S[(unsigned long)(unsigned)((hole(H1, u) * no + hole(H2, w)) * nv + g1) * ld + g2];
     }
 #pragma unroll
@@ -868,7 +882,7 @@ __device__ __forceinline__ Denominator denominator(cptr<FusedArgs> A, const Item
 __device__ __forceinline__ void phase() { __builtin_amdgcn_sched_barrier(0); }
 
 // v[r] = f(i, j, k, r), r = 16 i + 4 j + k, over the lane's elements, 0 in the
-// hole pairs (j, k) past a ragged edge.
+// hole pairs (j, k) without an element that counts.
 template <class F>
 __device__ __forceinline__ void each_element(const ItemGeo &G, double (&v)[64], F &&f) {
 #pragma unroll
@@ -877,7 +891,7 @@ __device__ __forceinline__ void each_element(const ItemGeo &G, double (&v)[64], 
     for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii) v[16 * ii + 4 * jj + kk] = 0.0;
-      if (jj < G.J.n && kk < G.K.n)
+      if (G.pair(0, jj, kk))
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii)
           v[16 * ii + 4 * jj + kk] = f(ii, jj, kk, 16 * ii + 4 * jj + kk);
@@ -900,14 +914,14 @@ __device__ __forceinline__ void each_element_with(const ItemGeo &G, gptr<const d
     if (jj < G.J.n)
 #pragma unroll
       for (int n = 0; n < 16; ++n)
-        if ((n & 3) < G.K.n) v[16 * (n >> 2) + 4 * jj + (n & 3)] = f(n >> 2, jj, n & 3, x[n]);
+        if (G.pair(0, jj, n & 3)) v[16 * (n >> 2) + 4 * jj + (n & 3)] = f(n >> 2, jj, n & 3, x[n]);
     phase();
   }
 }
 
 // f(r, factor of the singles product of element r) over the 9 singles
 // products of the lane's elements, r = 16 i + 4 j + k, from the staged
-// operands; the elements of one hole pair past a ragged edge are skipped.
+// operands; hole pairs without an element that counts are skipped.
 template <class F>
 __device__ __forceinline__ void each_single(const double *e, const ItemGeo &G, const Place &p,
                                             F &&f) {
@@ -924,12 +938,11 @@ __device__ __forceinline__ void each_single(const double *e, const ItemGeo &G, c
       tc[u] = t1[((2 * 3 + t) * 8 + sc) * 4 + u];
     }
     const double sg = t == 1 ? -1.0 : 1.0;
-    const int n1 = t == 0 ? G.J.n : G.I.n, n2 = t == 2 ? G.J.n : G.K.n;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        if (!(u < n1 && w < n2)) continue;
+        if (!G.pair(t, u, w)) continue;
         const double *sp = e + (t * 16 + u * 4 + w) * 192;
         const double sbc = sg * sp[obc], sac = sg * sp[oac], sab = sg * sp[oab];
 #pragma unroll
@@ -952,12 +965,12 @@ __device__ __forceinline__ void energy(const Q (&q)[16], const double *e, cptr<F
   e5 = 0.0;
   if (!inside(T, p)) return;
   const Denominator D = denominator(A, G, p);
-  const double factor = T->factor;
+  const double factor = T->factor * G.distinct();
   double den[64];
   each_element(G, den, [&](int ii, int jj, int kk, int) {
     const double d = (double)q[4 * jj + kk][ii];
     const double dn = d * factor / (D.eh[0][ii] + D.eh[1][jj] + D.eh[2][kk] + D.d0);
-    const bool ok = ii < G.I.n;
+    const bool ok = G.pair(2, ii, jj);
     e4 += ok ? dn * d : 0.0;
     return ok ? dn : 0.0;
   });
@@ -1061,12 +1074,12 @@ __device__ __forceinline__ void lambda_right(const Q (&q)[16], const double *e, 
   e2 = 0.0;
   if (!inside(T, p)) return;
   const Denominator D = denominator(A, G, p);
-  const double factor = T->factor;
+  const double factor = T->factor * G.distinct();
   double den[64];
   each_element_with(G, in, lane, den, [&](int ii, int jj, int kk, double yd) {
     const double dn = (double)q[4 * jj + kk][ii] * factor /
                       (D.eh[0][ii] + D.eh[1][jj] + D.eh[2][kk] + D.d0);
-    const bool ok = ii < G.I.n;
+    const bool ok = G.pair(2, ii, jj);
     e1 += ok ? dn * yd : 0.0;
     return ok ? dn : 0.0;
   });
@@ -1088,11 +1101,11 @@ __device__ __forceinline__ void cr_right(const Q (&q)[16], const double *e, cptr
   s[0] = s[1] = s[2] = s[3] = 0.0;
   if (!inside(T, p)) return;
   const Denominator D = denominator(A, G, p);
-  const double factor = T->factor;
+  const double factor = T->factor * G.distinct();
   double d0 = D.d0;
   auto weight = [&](int ii, int jj, int kk) {
     const double w = factor / (D.eh[0][ii] + D.eh[1][jj] + D.eh[2][kk] + d0);
-    return ii < G.I.n ? w : 0.0;
+    return G.pair(2, ii, jj) ? w : 0.0;
   };
   // the accumulators are read out first, then one 64-value array is live at a
   // time (both together do not fit the registers; a third division is cheaper)
@@ -1108,7 +1121,7 @@ __device__ __forceinline__ void cr_right(const Q (&q)[16], const double *e, cptr
     if (jj < G.J.n)
 #pragma unroll
       for (int n = 0; n < 16; ++n)
-        if ((n & 3) < G.K.n) {
+        if (G.pair(0, jj, n & 3)) {
           const double rd = (double)q[4 * jj + (n & 3)][n >> 2] * weight(n >> 2, jj, n & 3);
           s[0] += rd * td[n];
           s[1] += rd * ts[n];
@@ -1148,7 +1161,10 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
   // (every barrier is reached by all 8 waves): the dynamic schedule of
   // sched_item when `sched` is given, else a static round-robin.
   const bool dyn = sched != nullptr;
-  const int sh = (dyn ? (int)sched[9] : 0) + (HALF ? 1 : 0);  // log2 of the slice width
+  // log2 of the slice width; a launch of fewer than eight slices takes narrower
+  // ones, so that every XCD has items of its own
+  int sh = (dyn ? (int)sched[9] : 0) + (HALF ? 1 : 0);
+  while (sh > 0 && (8l << sh) > nglobal) --sh;
   unsigned queue = blockIdx.x & 7u;  // thread 0: the queue it draws from
   unsigned long long ticket = 0;
   long g = 0;
@@ -1192,6 +1208,7 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
     G.J = hbox(T->oh2, bj, T->r2);
     G.K = hbox(T->oh3, bk, T->r3);
     auto prng = [](int o, int r, int n) { return PRange{o, min(n - 1, r - 1), 0}; };
+    G.heq = T->eq & (EQ_IJ | EQ_JK);
     G.a = prng(T->op4 + 8 * ba, T->r4 - 8 * ba, 8);
     G.b = prng(T->op5 + 8 * bb, T->r5 - 8 * bb, 8);
     G.c = prng(T->op6 + 8 * bc + c4, T->r6 - 8 * bc - c4, HALF ? 4 : 8);
