@@ -1177,8 +1177,6 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
   for (long r = 0;; ++r) {
     if (dyn) {
       if (g < 0) break;
-      // the next item's ticket is drawn now and read at the end of this item
-      if (tid == 0) ticket = atomicAdd(&sched[queue], 1ull);
     } else {
       if (r * (long)gridDim.x >= nglobal) break;
       g = round_item(r, blockIdx.x, gridDim.x, nseg > 1);
@@ -1244,6 +1242,16 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
     const gptr<double> partials = (gptr<double>)A->partials;
     const gptr<double> den = (gptr<double>)M->cr_den;
     const bool empty = HALF && G.c.sm < 0;  // a half past the edge: no element
+    // The next item's ticket is drawn before this one's epilogue and read at its
+    // end.  Drawn at the start of the item, the first workgroups of a launch
+    // with fewer items than workgroups took two items each (no=8/nv=32, 160
+    // half items: 134 us, now 104), and the last round of a longer one was less
+    // even (CR no=16/nv=72 4.76 / 4.61 ms, Lambda no=20/nv=80 15.3 / 15.2).
+    // (The order of the tests here and below is the faster one of each kernel, all
+    // of which sit at the register limit: `dyn` first, no=40/nv=160 461 ms and a
+    // tile export of no=24/nv=96 1.28 ms; `dyn` second, 465 and 1.18 ms.)
+    if (EPI == EPI_TILES ? empty && dyn && tid == 0 : dyn && empty && tid == 0)
+      ticket = atomicAdd(&sched[queue], 1ull);
     if (empty && EPI != EPI_TILES && lane == 0) {
       partials[2 * part] = partials[2 * part + 1] = 0.0;
       if (EPI == EPI_CR) den[2 * part] = den[2 * part + 1] = 0.0;
@@ -1257,6 +1265,8 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
       typename Pr::quad q[16];
       contract<PREC>(q, lds, lds_base, MS, T, G, P, wave, lane);
       // Epilogue: the chunk buffers are free.
+      if (EPI == EPI_TILES ? side == 1 && dyn && tid == 0 : dyn && side == 1 && tid == 0)
+        ticket = atomicAdd(&sched[queue], 1ull);
       const long slot = ((long)blockIdx.x * NW + wave) * (EPI == EPI_CR ? 8192 : 4096);
       const gptr<double> spill = (gptr<double>)M->spill + slot;
       const bool fock = EPI == EPI_LAMBDA && side == 0 && ML->lam_f != nullptr;
