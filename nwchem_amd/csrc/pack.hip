@@ -271,13 +271,16 @@ struct Runs {
 
 // Host ranges to the device.  The referenced ranges of a file form one stream
 // of R.total doubles (the runs in order, at device offsets base[k]); the
-// streams are cut into pieces of 1 MiB, which the host threads take in turn:
-// each gathers a piece into one of its two pinned buffers and queues that
-// buffer's copy, so gathers and DMA overlap throughout and the pinned memory,
-// 32 MiB at most, stays in the host's caches.  Two pinned buffers of 64 MiB,
-// each filled by 16 threads started for it, took 5.5 of the 7.7 ms of an
-// upload of 74 MB in three files at no=20/nv=80, whose DMA takes 1.5; the upload
-// now takes 3.7 (pieces of 2 MiB 5.9, 8 threads 4.5 to 5.8).
+// streams are cut into pieces.  Up to 256 MiB in all (small()), the pieces are of
+// 1 MiB and the host threads take them in turn: each gathers a piece into one
+// of its two pinned buffers and queues that buffer's copy, so gathers and DMA
+// overlap throughout and the pinned memory, 32 MiB at most, stays in the host's
+// caches.  Above, all threads together gather a piece of 64 MiB into one of two
+// pinned buffers while the DMA of the other runs (large()).  Measured at 74 MB
+// (no=20/nv=80, DMA alone 1.5 ms): large 7.7 ms, of which threads started for
+// each buffer and the pinning of 128 MiB take half, small 3.7; no=8/nv=32 2.2
+// and 0.5 ms; at 1.9 GB (no=40/nv=160), where the DMA bounds both, large 38 ms,
+// small 45 (copies of 4 MiB 40, 8 MiB 41).
 class Upload {
  public:
   Upload(int device, hipStream_t stream, char *dst) : device_(device), stream_(stream), dst_(dst) {}
@@ -290,23 +293,38 @@ class Upload {
   }
   // the runs R of `file`, to dst + at on the device; R and file live until the
   // copies complete
-  void add(const Runs &R, const double *file, size_t at) {
-    for (long p = 0; p < R.total; p += PIECE)
-      pieces_.push_back({&R, file, p, std::min(PIECE, R.total - p), at + (size_t)p * sizeof(double)});
-  }
+  void add(const Runs &R, const double *file, size_t at) { files_.push_back({&R, file, 0, R.total, at}); }
   // Queues every piece on the stream; the first error of any thread.
   hipError_t start() {
+    long total = 0;
+    for (const Piece &f : files_) total += f.n;
+    piece_ = total <= SMALL ? 1l << 17 : 1l << 23;
+    for (const Piece &f : files_)
+      for (long p = 0; p < f.n; p += piece_)
+        pieces_.push_back({f.R, f.file, p, std::min(piece_, f.n - p), f.at + (size_t)p * sizeof(double)});
     const long np = (long)pieces_.size();
     if (np == 0) return hipSuccess;
     const long nt = std::min({np, 16l, std::max(1l, (long)std::thread::hardware_concurrency())});
-    const long slots = std::min(np, 2 * nt);
-    hipError_t e = hipHostMalloc((void **)&stage_, slots * PIECE * sizeof(double));
+    const long slots = total <= SMALL ? std::min(np, 2 * nt) : 2;
+    hipError_t e = hipHostMalloc((void **)&stage_, slots * piece_ * sizeof(double));
     for (long k = 0; k < slots && e == hipSuccess; ++k) {
       hipEvent_t x;
       e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
       if (e == hipSuccess) ev_.push_back(x);
     }
     if (e != hipSuccess) return e;
+    return total <= SMALL ? small(nt, slots) : large(nt);
+  }
+
+ private:
+  static constexpr long SMALL = 1l << 25;  // doubles
+  struct Piece {
+    const Runs *R;
+    const double *file;
+    long p0, n;  // stream positions
+    size_t at;
+  };
+  hipError_t small(long nt, long slots) {
     std::vector<std::thread> th;
     try {
       for (long t = 1; t < nt; ++t) th.emplace_back([this, t, nt, slots] { work(t, nt, slots); });
@@ -318,14 +336,6 @@ class Upload {
     return (hipError_t)error_.load();
   }
 
- private:
-  static constexpr long PIECE = 1l << 17;  // doubles
-  struct Piece {
-    const Runs *R;
-    const double *file;
-    long p0, n;  // stream positions
-    size_t at;
-  };
   // Thread t of nt: slots t and t + nt (the second one if there is one).
   void work(long t, long nt, long slots) {
     hipError_t e = hipSetDevice(device_);
@@ -334,7 +344,7 @@ class Upload {
       const long k = next_.fetch_add(1);
       if (k >= (long)pieces_.size()) return;
       const long slot = t + (done % mine) * nt;
-      double *buf = stage_ + slot * PIECE;
+      double *buf = stage_ + slot * piece_;
       // the copy that last read this buffer must be done
       if (done >= mine) e = hipEventSynchronize(ev_[slot]);
       if (e != hipSuccess) break;
@@ -344,6 +354,33 @@ class Upload {
       if (e == hipSuccess) e = hipEventRecord(ev_[slot], stream_);
     }
     if (e != hipSuccess) error_.store(e);
+  }
+  hipError_t large(long nt) {
+    for (size_t k = 0; k < pieces_.size(); ++k) {
+      const Piece &p = pieces_[k];
+      double *buf = stage_ + (long)(k & 1) * piece_;
+      hipError_t e = k >= 2 ? hipEventSynchronize(ev_[k & 1]) : hipSuccess;
+      if (e != hipSuccess) return e;
+      const long part = (p.n + nt - 1) / nt;
+      auto share = [&](long t) {
+        const long at = t * part, n = std::min(part, p.n - at);
+        if (n > 0) gather({p.R, p.file, p.p0 + at, n, 0}, buf + at);
+      };
+      std::vector<std::thread> th;
+      long t = 1;
+      try {
+        for (; t < nt; ++t) th.emplace_back(share, t);
+      } catch (const std::system_error &) {
+        // this thread takes the shares of those that could not be started
+      }
+      for (; t < nt; ++t) share(t);
+      share(0);
+      for (auto &x : th) x.join();
+      e = hipMemcpyAsync(dst_ + p.at, buf, p.n * sizeof(double), hipMemcpyHostToDevice, stream_);
+      if (e == hipSuccess) e = hipEventRecord(ev_[k & 1], stream_);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
   }
   static void gather(const Piece &p, double *dst) {
     const Runs &R = *p.R;
@@ -359,7 +396,8 @@ class Upload {
   int device_;
   hipStream_t stream_;
   char *dst_;
-  std::vector<Piece> pieces_;
+  long piece_ = 0;  // doubles of a piece
+  std::vector<Piece> files_, pieces_;
   std::vector<hipEvent_t> ev_;
   double *stage_ = nullptr;
   std::atomic<long> next_{0};
