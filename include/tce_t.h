@@ -326,10 +326,10 @@ int tce_t_job_upload_lambda(tce_t_job *job, const double *y1, const long *k_y1_o
  *   energy2 += factor * tdoubles * (ysingles + ydoubles) / D
  * task_energies (2 * ntasks doubles, or NULL) receives {energy1, energy2}
  * of each task in loop order.  Synchronous.  Device memory: the orbital
- * pairing (same tiling on both jobs, not TCE_T_TILING_ORBITAL) runs two
- * passes of the contraction kernel over the jobs' kernel tasks with a
- * window of at most 16 GiB (a quarter of the free memory) allocated for
- * the call; the reference order (and ORBITAL-tiled jobs) keep each job's
+ * pairing (same tiling on both jobs, not TCE_T_TILING_ORBITAL) runs one
+ * launch of the contraction kernel over the jobs' kernel tasks with 64 MiB
+ * of spill slots, which the right-hand job allocates once and keeps; the
+ * reference order (and ORBITAL-tiled jobs) keep each job's
  * tile buffer, 16 bytes per element of the largest task tile, as
  * tce_t_job_triples_tiles does. */
 int tce_t_lambda_ccsd_t(tce_t_job *right, tce_t_job *left, const double *f1,
@@ -364,8 +364,8 @@ int tce_t_job_upload_cr(tce_t_job *job, const double *t1, const long *k_t1_offse
  * den0 = the overlap of cr_ccsd_t_D with c = t, and
  *   energy1 = num1 / (1 + den1 + den0), energy2 = num2 / (1 + den2 + den0).
  * terms (5 doubles or NULL) receives num1, num2, den0, den1, den2.
- * Synchronous; two passes of the contraction kernel with the window of
- * tce_t_lambda_ccsd_t. */
+ * Synchronous; one launch of the contraction kernel with 128 MiB of spill
+ * slots, which the cr job allocates once and keeps. */
 int tce_t_cr_ccsd_t(tce_t_job *triples, tce_t_job *cr, int precision, double *energy1,
                     double *energy2, double *terms);
 /* Host packer of tce_t_job_upload, for inspection and tests: the dense tensors

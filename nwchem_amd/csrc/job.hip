@@ -200,7 +200,7 @@ extern "C" int tce_t_init(int device) {
   return TCE_T_OK;
 }
 
-// Contraction ranges of the 18 passes of fused_mixed (TaskDev::x0/x1) for a
+// Contraction ranges of the 18 passes of fused_mixed (TaskDev::x) for a
 // task with tiles (p4b, p5b, p6b, h1b, h2b, h3b): the hull of the orbitals
 // whose spin and irrep the pass's blocks allow, in the occupied (d1) or
 // virtual (d2) space.  The reference applies the same spin and irrep tests
