@@ -11,8 +11,8 @@
 //
 // Differences in mechanism (not in results): one library stream instead of a
 // stream created and destroyed per call; operands staged through a reusable
-// pinned buffer; one generic kernel per family (d1, d2, s1) parameterised by
-// the output permutation of the variant instead of 25 hand-expanded kernels;
+// pinned buffer; one contraction kernel parameterised by the strides of the
+// family (d1, d2, s1) and variant instead of 25 hand-expanded kernels;
 // a two-pass deterministic energy reduction instead of one-thread blocks and a
 // host-side sum.  Errors are recorded (tce_t_last_error) and reported on
 // stderr rather than calling exit(1).
