@@ -80,6 +80,7 @@
 #include <type_traits>
 
 #include "fused.h"
+#include "handover.h"
 
 namespace tce_t {
 namespace {
@@ -1186,7 +1187,7 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
                                                            long nglobal,
                                                            unsigned long long *sched) {
   __shared__ f4 lds[lds_quads<PREC>()];
-  __shared__ long next_item;  // dynamic schedule: the workgroup's next item
+  __shared__ NextItem next_item;  // dynamic schedule: the workgroup's next item
   using Pr = Prec<PREC>;
   constexpr int NW = Pr::NW;
   constexpr bool HALF = NW == 4;  // the launch's indices are half items
@@ -1195,9 +1196,10 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
   const unsigned lds_base =
       (unsigned)uniform((int)(unsigned long)(__attribute__((address_space(3))) f4 *)lds);
   const cptr<MixedSegment> segs = (cptr<MixedSegment>)segments;
-  // Persistent loop over the launch's items, uniform across the workgroup
-  // (every barrier is reached by all 8 waves): the dynamic schedule of
-  // sched_item when `sched` is given, else a static round-robin.
+  // Persistent loop over the launch's items: the dynamic schedule of sched_item
+  // when `sched` is given, else a static round-robin.  The item is uniform
+  // across the workgroup, so its waves (4 or 8) reach the same barriers; an
+  // empty half has only the one at the item's end.
   const bool dyn = sched != nullptr;
   // log2 of the slice width; a launch of fewer than eight slices takes narrower
   // ones, so that every XCD has items of its own
@@ -1207,9 +1209,10 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
   unsigned long long ticket = 0;
   long g = 0;
   if (dyn) {
-    if (tid == 0) next_item = sched_item(sched, queue, atomicAdd(&sched[queue], 1ull), nglobal, sh);
+    if (tid == 0)
+      next_item.put(-1, sched_item(sched, queue, atomicAdd(&sched[queue], 1ull), nglobal, sh));
     __syncthreads();
-    g = uniform(next_item);
+    g = uniform(next_item.get(-1));
   }
   int seg = 0;  // segment of the workgroup's current item
   for (long r = 0;; ++r) {
@@ -1349,9 +1352,9 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
         }
       }
     }
-    if (dyn && tid == 0) next_item = sched_item(sched, queue, ticket, nglobal, sh);
+    if (dyn && tid == 0) next_item.put(r, sched_item(sched, queue, ticket, nglobal, sh));
     __syncthreads();  // the next item's first loads overwrite the staged data
-    if (dyn) g = uniform(next_item);
+    if (dyn) g = uniform(next_item.get(r));
   }
   if (dyn && tid == 0) sched_leave(sched);
 }
