@@ -364,8 +364,8 @@ int tce_t_job_upload_cr(tce_t_job *job, const double *t1, const long *k_t1_offse
  * den0 = the overlap of cr_ccsd_t_D with c = t, and
  *   energy1 = num1 / (1 + den1 + den0), energy2 = num2 / (1 + den2 + den0).
  * terms (5 doubles or NULL) receives num1, num2, den0, den1, den2.
- * Synchronous; one launch of the contraction kernel with 128 MiB of spill
- * slots, which the cr job allocates once and keeps. */
+ * Synchronous; one launch of the contraction kernel with 96 MiB (FP64 128
+ * MiB) of spill slots, which the cr job allocates once and keeps. */
 int tce_t_cr_ccsd_t(tce_t_job *triples, tce_t_job *cr, int precision, double *energy1,
                     double *energy2, double *terms);
 /* Host packer of tce_t_job_upload, for inspection and tests: the dense tensors

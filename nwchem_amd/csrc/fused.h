@@ -407,8 +407,10 @@ int launch_fused_tiles(const MixedSegment *segs, long total, int precision, int 
 // denominator tile into args->cr_den.
 int launch_fused_pair(const MixedSegment *segs, long total, int precision, int grid, hipStream_t s,
                       unsigned long long *sched, bool cr);
-// Doubles of one workgroup's slot of MixedArgs::spill.
-constexpr long pair_slot_doubles(bool cr) { return cr ? 8L * 8192 : 8L * 4096; }
+// Doubles of one wave's and of one 8-wave group's slot of MixedArgs::spill: 64
+// values a lane; CR 128, the first 64 as FP32 where the accumulators are (f32).
+constexpr long pair_wave_doubles(bool cr, bool f32) { return cr ? (f32 ? 6144 : 8192) : 4096; }
+constexpr long pair_slot_doubles(bool cr, bool f32) { return 8 * pair_wave_doubles(cr, f32); }
 // Zeroed counters of the dynamic schedule for one launching stream (every
 // launch leaves them zero; launches that may overlap need their own), or
 // null on failure (error set).  Free with hipFree.

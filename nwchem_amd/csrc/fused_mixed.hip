@@ -899,7 +899,40 @@ __device__ __forceinline__ void each_element(const ItemGeo &G, double (&v)[64], 
     }
 }
 
-// The same with the element's value x in the spill slot: v[r] = f(i, j, k, x),
+// Between the two halves of an item the wave's left-hand values wait in its
+// slot of a spill buffer, element r = 16 i + 4 j + k of the lane at [r * 64 +
+// lane]; CR: the doubles so, as FP32 where the accumulators are (their exact
+// values), the singles behind them.  A slot belongs to a workgroup, not to an
+// item: 64 MB for 256 workgroups, CR 128 MB in FP64 and 96 MB in the other modes.
+// One slot per item of a window of up to 16 GB, written by a launch over the
+// left-hand job and read by one over the right-hand job, cost the allocation of
+// the window on each call (45 to 300 ms for the call at no=20/nv=80, 53 ms at
+// no=16/nv=72, of which the kernels took 45 and 7.7 ms) and two passes over it
+// in HBM.
+// What the slots cost is not their own time but the operands they push out of
+// the caches: with 64-bit doubles and ordinary accesses a CR item's bf16x3
+// contractions at no=40/nv=160 took 258k clocks a side, 186k without the slot
+// accesses (the FP64 mode's, 742k, change by 1%).  FP32 doubles bring 193k, and
+// accesses marked as streaming 187k.  CR before / now (two launches over a
+// window), s: bf16x3 no=40/nv=160 0.351 / 0.275 (0.333), no=40/nv=320 4.19 / 3.34
+// (3.60); bf16x6 0.486 / 0.419 (0.509) and 6.14 / 5.47 (5.97).
+template <class T, class V>
+__device__ __forceinline__ void slot_put(gptr<T> slot, int r, int lane, V v) {
+  __builtin_nontemporal_store((T)v, &slot[r * 64 + lane]);
+}
+template <class T>
+__device__ __forceinline__ T slot_get(gptr<const T> slot, int r, int lane) {
+  return __builtin_nontemporal_load(&slot[r * 64 + lane]);
+}
+// The CR doubles' type in the slot, and the singles' place behind them.
+template <class Q>
+using slot_t = std::conditional_t<sizeof(Q) == 16, float, double>;
+template <class T>
+constexpr int singles_at() {
+  return 64 * 64 * (int)sizeof(T) / 8;
+}
+
+// each_element with the element's value x in the slot: v[r] = f(i, j, k, x),
 // read 16 at a time (one wait each, not one per hole pair).
 template <class F>
 __device__ __forceinline__ void each_element_with(const ItemGeo &G, gptr<const double> in, int lane,
@@ -910,7 +943,7 @@ __device__ __forceinline__ void each_element_with(const ItemGeo &G, gptr<const d
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
       v[16 * (n >> 2) + 4 * jj + (n & 3)] = 0.0;
-      x[n] = in[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
+      x[n] = slot_get(in, 16 * (n >> 2) + 4 * jj + (n & 3), lane);
     }
     if (jj < G.J.n)
 #pragma unroll
@@ -1022,16 +1055,6 @@ __device__ __forceinline__ void store_tiles(const Q (&q)[16], const double *e, c
 enum { EPI_ENERGY = 0, EPI_TILES = 1, EPI_LAMBDA = 2, EPI_CR = 3 };
 constexpr bool pair_epilogue(int epi) { return epi == EPI_LAMBDA || epi == EPI_CR; }
 
-// Between the two halves of an item the wave's left-hand values wait in its
-// slot of a spill buffer, element r = 16 i + 4 j + k of the lane at out[r * 64 +
-// lane] (CR: the singles at out[(64 + r) * 64 + lane]).  A slot belongs to a
-// workgroup, not to an item: 64 MB (CR 128 MB) for 256 workgroups, which the
-// caches hold.  One slot per item of a window of up to 16 GB, written by a
-// launch over the left-hand job and read by one over the right-hand job, cost
-// the allocation of the window on each call (45 to 300 ms for the call at
-// no=20/nv=80, 53 ms at no=16/nv=72, of which the kernels took 45 and 7.7 ms)
-// and two passes over it in HBM.
-
 // Left-hand half of a Lambda item: the y3 doubles, i.e. the accumulators plus
 // the Fock term P(c/ab) P(k/ij) y(a b i j) f(k c).  Written out, that term is
 // the singles term with f(h p) for t1(p h) and y(p p' h h') for S: its operands
@@ -1046,7 +1069,7 @@ __device__ __forceinline__ void lambda_left(const Q (&q)[16], const double *e, b
   for (int r = 0; r < 64; ++r) yd[r] = (double)q[r & 15][r >> 4];
   if (fock) each_single(e, G, p, [&](int r, double s) { yd[r] += s; });
 #pragma unroll
-  for (int r = 0; r < 64; ++r) out[r * 64 + lane] = yd[r];
+  for (int r = 0; r < 64; ++r) slot_put(out, r, lane, yd[r]);
 }
 
 // Left-hand half of a CR item: the t3 doubles and singles.
@@ -1054,12 +1077,12 @@ template <class Q>
 __device__ __forceinline__ void cr_left(const Q (&q)[16], const double *e, const Place &p,
                                         const ItemGeo &G, gptr<double> out, int lane) {
 #pragma unroll
-  for (int r = 0; r < 64; ++r) out[r * 64 + lane] = (double)q[r & 15][r >> 4];
+  for (int r = 0; r < 64; ++r) slot_put((gptr<slot_t<Q>>)out, r, lane, q[r & 15][r >> 4]);
   phase();
   double sv[64];
   singles_products(e, G, p, sv);
 #pragma unroll
-  for (int r = 0; r < 64; ++r) out[(64 + r) * 64 + lane] = sv[r];
+  for (int r = 0; r < 64; ++r) slot_put(out + singles_at<slot_t<Q>>(), r, lane, sv[r]);
 }
 
 // Right-hand half of a Lambda item: den = t3d * factor / D as in energy(), e1
@@ -1112,7 +1135,8 @@ __device__ __forceinline__ void cr_right(const Q (&q)[16], const double *e, cptr
   // slot and 64 divisions instead of two and 192 (no=40/nv=160, bf16x6 566 / 484
   // ms, bf16x3 430 / 353, FP32 634 / 577).
   if constexpr (sizeof(q[0][0]) == 4) {
-    const gptr<const double> in2 = in + 64 * 64;
+    const gptr<const slot_t<Q>> in1 = (gptr<const slot_t<Q>>)in;
+    const gptr<const double> in2 = in + singles_at<slot_t<Q>>();
     double sv[64];
     singles_products(e, G, p, sv);
     phase();
@@ -1124,8 +1148,8 @@ __device__ __forceinline__ void cr_right(const Q (&q)[16], const double *e, cptr
 #pragma unroll
         for (int n = 0; n < 8; ++n) {
           const int r = 16 * (i0 + (n >> 2)) + 4 * jj + (n & 3);
-          td[n] = in[r * 64 + lane];
-          ts[n] = in2[r * 64 + lane];
+          td[n] = slot_get(in1, r, lane);
+          ts[n] = slot_get(in2, r, lane);
         }
         if (jj < G.J.n)
 #pragma unroll
@@ -1148,14 +1172,14 @@ __device__ __forceinline__ void cr_right(const Q (&q)[16], const double *e, cptr
   }
   // the accumulators are read out first, then one 64-value array is live at a
   // time (both together do not fit the registers; a third division is cheaper)
-  const gptr<const double> ins = in + 64 * 64;
+  const gptr<const double> ins = in + singles_at<slot_t<Q>>();
 #pragma unroll
   for (int jj = 0; jj < 4; ++jj) {
     double td[16], ts[16];
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
-      td[n] = in[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
-      ts[n] = ins[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
+      td[n] = slot_get(in, 16 * (n >> 2) + 4 * jj + (n & 3), lane);
+      ts[n] = slot_get(ins, 16 * (n >> 2) + 4 * jj + (n & 3), lane);
     }
     if (jj < G.J.n)
 #pragma unroll
@@ -1308,7 +1332,8 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
       // Epilogue: the chunk buffers are free.
       if (EPI == EPI_TILES ? side == 1 && dyn && tid == 0 : dyn && side == 1 && tid == 0)
         ticket = atomicAdd(&sched[queue], 1ull);
-      const long slot = ((long)blockIdx.x * NW + wave) * (EPI == EPI_CR ? 8192 : 4096);
+      const long slot = ((long)blockIdx.x * NW + wave) *
+                        pair_wave_doubles(EPI == EPI_CR, PREC != TCE_T_FP64);
       const gptr<double> spill = (gptr<double>)M->spill + slot;
       const bool fock = EPI == EPI_LAMBDA && side == 0 && ML->lam_f != nullptr;
       if (fock)

@@ -185,7 +185,8 @@ int lambda_fused(Job &JR, Job &JL, const double *dF, int precision, std::vector<
     int cus = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, JR.device), "attr");
     const int grid = (int)std::min<long>(std::max(1, cus), N);
-    const size_t need = (size_t)grid * pair_slot_doubles(cr_den != nullptr) * sizeof(double);
+    const size_t need =
+        (size_t)grid * pair_slot_doubles(cr_den != nullptr, precision != TCE_T_FP64) * sizeof(double);
     if (JR.dspill_bytes < need) {
       if (JR.dspill) HIPCHK(hipFree(JR.dspill), "spill slots");
       JR.dspill = nullptr;
