@@ -518,7 +518,10 @@ void launch_call(int family, int n, const long dims[6], long K, const double *ha
 // as in ccsd_t_dot.F:89-110; first pass: one partial pair per block.  The
 // orbital energies of the six tiles are e1..e6 (h1, h2, h3, p4, p5, p6).
 // A unit of work is one particle triple by up to kEnChunk elements of its
-// hole block, whose e_h1 + e_h2 + e_h3 sit in LDS.
+// hole block, whose e_h1 + e_h2 + e_h3 sit in LDS; where the hole block leaves
+// half of the threads idle or more, as many triples as the threads hold (a
+// single hole orbital, 64 particles each: one triple at a time 259 us for the
+// call, 256 at a time 32; one element a thread in turn 115).
 // Bound: HBM, 16 bytes per element.  With five 64-bit divisions per element to
 // find its indices, 24e6 elements took 147 us; their bytes take 82 us.
 constexpr int kEnChunk = 2048;
@@ -534,11 +537,14 @@ __device__ __forceinline__ void energy_block(long h1d, long h2d, long h3d, long 
                                              double *__restrict__ part) {
   __shared__ double eh[kEnChunk];
   const long F = h1d * h2d * h3d, P = p4d * p5d * p6d;
-  const long units = (F + kEnChunk - 1) / kEnChunk * P;
+  const int per = F > 0 && F <= 128 ? 256 / (int)F : 1;  // triples of a unit
+  const int mine = per > 1 ? (int)threadIdx.x / (int)F : 0;
+  const int first = (int)threadIdx.x - mine * (int)F, step = per > 1 ? (int)F : 256;
+  const long groups = (P + per - 1) / per, units = (F + kEnChunk - 1) / kEnChunk * groups;
   double s1 = 0.0, s2 = 0.0;
   long cur = -1;
   for (long u = blockIdx.x; u < units; u += gridDim.x) {
-    const long chunk = u / P, pt = u - chunk * P, f0 = chunk * kEnChunk;
+    const long chunk = u / groups, pt = (u - chunk * groups) * per + mine, f0 = chunk * kEnChunk;
     const int n = (int)(F - f0 < kEnChunk ? F - f0 : kEnChunk);
     if (chunk != cur) {  // uniform
       __syncthreads();
@@ -549,11 +555,12 @@ __device__ __forceinline__ void energy_block(long h1d, long h2d, long h3d, long 
       __syncthreads();
       cur = chunk;
     }
+    if (mine >= per || pt >= P) continue;  // groups share the one chunk: no barrier ahead
     const long p45 = pt / p6d;
     const double denom_0 = -(e4[p45 / p5d] + e5[p45 % p5d] + e6[pt - p45 * p6d]);
     const double *d = t3d + pt * F + f0, *s = t3s + pt * F + f0;
 #pragma unroll 4
-    for (int f = threadIdx.x; f < n; f += 256) {
+    for (int f = first; f < n; f += step) {
       const double doub = d[f], sing = s[f];
       const double denom = doub * factor / (eh[f] + denom_0);
       s1 += denom * doub;
