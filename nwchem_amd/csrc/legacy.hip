@@ -11,11 +11,11 @@
 //
 // Differences in mechanism (not in results): one library stream instead of a
 // stream created and destroyed per call; operands staged through a reusable
-// pinned buffer; one contraction kernel parameterised by the strides of the
-// family (d1, d2, s1) and variant instead of 25 hand-expanded kernels;
-// a two-pass deterministic energy reduction instead of one-thread blocks and a
-// host-side sum.  Errors are recorded (tce_t_last_error) and reported on
-// stderr rather than calling exit(1).
+// pinned buffer; one contraction kernel, and one for small calls, parameterised
+// by the strides of the family (d1, d2, s1) and variant instead of 25
+// hand-expanded kernels; a two-pass deterministic energy reduction instead of
+// one-thread blocks and a host-side sum.  Errors are recorded (tce_t_last_error)
+// and reported on stderr rather than calling exit(1).
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
@@ -325,6 +325,58 @@ __global__ void __launch_bounds__(256) contract_kernel(DirectArgs c, double *__r
         t[u * c.a_t + v * c.b_t] = old[u][v] + c.sign * acc[u][v];
 }
 
+// The same with one element a thread, in t3's own order, on the operands as they
+// come: calls too small to fill the chip with tiles.
+__global__ void __launch_bounds__(256) contract_elements(CallArgs c, double *__restrict__ t3,
+                                                         const double *__restrict__ a,
+                                                         const double *__restrict__ b) {
+  const unsigned o = blockIdx.x * 256u + threadIdx.x;
+  if (o >= c.total) return;
+  unsigned r = o;
+  long oa = 0, ob = 0;
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    const unsigned n = (unsigned)c.dimL[q], v = r % n;
+    r /= n;
+    oa += v * c.sa[c.codeL[q]];
+    ob += v * c.sb[c.codeL[q]];
+  }
+  double acc = 0.0;
+  for (long k = 0; k < c.K; ++k) acc = fma(a[oa + k * c.ka], b[ob + k * c.kb], acc);
+  t3[o] += c.sign * acc;
+}
+
+// How a call runs.  Tiles pay from 2^20 elements (s1) or 2^22 multiply-adds
+// (d1, d2) on; below, their fewer threads and the packing launch cost more than
+// they save.  Time of a call, elements / tiles (h holes and p particles each,
+// contraction over one of them): s1 h=6,p=12 25.6 / 26.6 us, 10,10 29.8 / 28.6,
+// 8,16 39 / 31; d1 1,8 18.3 / 23.1, 6,12 28.4 / 31.6, 3,40 37.9 / 34.5, 10,10 41.2
+// / 37.8; d2 1,8 19 / 24, 3,16 30 / 35, 6,12 35.1 / 34.6, 5,16 48 / 38, 8,16 107 / 49.
+// Packing gains through the hole indices; a block of one hole triple has none
+// (d2 1,100 414 us packed, 405 not).  The tiled kernels count in 32 bits and put
+// one particle index in grid.y, which ends at 65535.
+struct Route {
+  bool tiled, pack;
+};
+Route route_of(const CallArgs &c, int family, long na, long nb) {
+  long x = 1, third = 1;
+  bool a = false, b = false;
+  for (int q = 0; q < 6; ++q) {
+    const bool on = q >= 3 && on_a(family, c.codeL[q]);
+    const bool tile = q >= 3 && (on ? !a : !b);
+    if (q >= 3 && !tile) third = c.dimL[q];
+    else x *= tile ? (c.dimL[q] + 3) / 4 : c.dimL[q];
+    if (q >= 3) (on ? a : b) = true;
+  }
+  const long most = 0xffffff00l;
+  Route r;
+  r.tiled = c.total * std::max(c.K, 1l) >= (family == 0 ? 1l << 20 : 1l << 22) && third <= 65535 &&
+            x <= most;
+  r.pack = r.tiled && family != 0 && c.K > 0 && c.dimL[0] * c.dimL[1] * c.dimL[2] > 1 &&
+           na <= most && nb <= most;
+  return r;
+}
+
 // TTGT back end (the alternative of sd_t_total_ttlg.cu: GEMM plus
 // transposes): the d1/d2 contraction as one DGEMM into C[m + M n] (rocBLAS,
 // FP64 matrix cores), m and n the output indices that sit on the t2 and the
@@ -424,9 +476,15 @@ void launch_call(int family, int n, const long dims[6], long K, const double *ha
   }
   memcpy(S.pinned, ha, na * sizeof(double));
   memcpy(S.pinned + na, hb, nb * sizeof(double));
-  // the direct d1/d2 contractions read packed copies behind the operands
-  const bool pack = family != 0 && backend_of(S) == TCE_T_LEGACY_DIRECT && K > 0;
-  double *dops = (double *)S.pool.get(pack ? 2 * bytes : bytes);
+  Route route = route_of(c, family, na, nb);
+  if (family != 0 && backend_of(S) != TCE_T_LEGACY_DIRECT) route.pack = false;
+  // packed copies go behind the operands
+  double *dops = (double *)S.pool.get(route.pack ? 2 * bytes : bytes);
+  if (!dops && route.pack) {
+    (void)hipGetLastError();
+    route.pack = false;
+    dops = (double *)S.pool.get(bytes);
+  }
   if (!dops) {
     set_error("device pool allocation failed");
     S.failed = true;
@@ -489,7 +547,7 @@ void launch_call(int family, int n, const long dims[6], long K, const double *ha
     if (!ok(hipGetLastError(), "permute_add_kernel launch")) return;
   } else {
     const double *ops = dops;
-    if (pack) {
+    if (route.pack) {
       PackPair P;
       P.p[0] = pack_args(c, family, true);
       P.p[1] = pack_args(c, family, false);
@@ -501,9 +559,14 @@ void launch_call(int family, int n, const long dims[6], long K, const double *ha
       if (!ok(hipGetLastError(), "pack_operands launch")) return;
       ops = packed;
     }
-    const DirectArgs da = direct_args(c, family);
-    hipLaunchKernelGGL(contract_kernel, dim3((da.threads + 255) / 256, da.nc), dim3(256), 0,
-                       S.stream, da, t3, ops, ops + na);
+    if (route.tiled) {
+      const DirectArgs da = direct_args(c, family);
+      hipLaunchKernelGGL(contract_kernel, dim3((da.threads + 255) / 256, da.nc), dim3(256), 0,
+                         S.stream, da, t3, ops, ops + na);
+    } else {
+      hipLaunchKernelGGL(contract_elements, dim3((unsigned)blocks), dim3(threads), 0, S.stream, c,
+                         t3, ops, ops + na);
+    }
     if (!ok(hipGetLastError(), "contract_kernel launch")) return;
   }
   if (host_t3 && !ok(hipMemcpyAsync(host_t3, t3, tbytes, hipMemcpyDeviceToHost, S.stream), "D2H t3"))

@@ -5,6 +5,13 @@ Energy (compute_en_): hole blocks of 1 to 129 and of 2049 elements (as many
 particle triples to a unit of work as 256 threads hold, two halves, one triple,
 two LDS chunks), particle counts that fill no unit or leave a remainder.
 Tolerance: max(1e-10, 1e-12 |E|), as for every FP64 energy.
+
+Contractions (sd_t_*): each of the 27 calls at extents on both sides of the
+rule that takes it to register tiles or to one element a thread: small, ragged
+against the 4 x 4 tiles, a hole block of one element (not packed) and a particle
+index longer than a grid's second dimension.
+Tolerance: K products summed in any order, (K + 2) 2^-53 sum |a b| + 2^-52 |t3|
+for every element.
 """
 import ctypes as C
 
@@ -57,3 +64,45 @@ def test_energy_of_small_hole_blocks(dims):
     w = 0.5 * t / D
     for got, want in zip(e, ((w * t).sum(), (w * (t + s)).sum())):
         assert abs(got - want) <= max(1e-10, 1e-12 * abs(want)), (got, want)
+
+
+# layouts (fastest first) and signs of the 27 calls, ccsd_t_kernels_omp.F:5-1198; operands, fastest first
+HOLES = {"s1": ("h3 h2 h1", "h3 h1 h2", "h1 h3 h2"), "d1": ("h3 h2 h1", "h3 h1 h2", "h1 h3 h2"),
+         "d2": ("h3 h2 h1", "h2 h1 h3", "h2 h3 h1")}
+PARTICLES = {"s1": ("p6 p5 p4", "p6 p4 p5", "p4 p6 p5"), "d1": ("p6 p5 p4", "p5 p4 p6", "p5 p6 p4"),
+             "d2": ("p6 p5 p4", "p6 p4 p5", "p4 p6 p5")}
+SIGN = {"s1": (1, -1, 1, -1, 1, -1, 1, -1, 1), "d1": (-1, 1, -1, -1, 1, -1, 1, -1, 1),
+        "d2": (-1, -1, 1, 1, 1, -1, -1, -1, 1)}
+OPERANDS = {"s1": ("p4 h1", "h3 h2 p6 p5"), "d1": ("x p4 p5 h1", "h3 h2 p6 x"),
+            "d2": ("x p4 h1 h2", "x h3 p6 p5")}
+LETTER = {"h1": "i", "h2": "j", "h3": "k", "p4": "a", "p5": "b", "p6": "c", "x": "x"}
+
+# h1 h2 h3 p4 p5 p6, contraction
+SIZES = [((3, 2, 4, 5, 3, 6), 3), ((5, 6, 7, 9, 10, 11), 4), ((5, 6, 7, 9, 10, 13), 24),
+         ((7, 8, 9, 10, 13, 17), 4), ((1, 1, 1, 37, 41, 43), 70),
+         ((1, 1, 1, 70000, 1, 1), 64), ((1, 1, 1, 1, 70000, 1), 64), ((1, 1, 1, 1, 1, 70000), 64)]
+
+
+@pytest.mark.parametrize("fam", ["s1", "d1", "d2"])
+@pytest.mark.parametrize("size", SIZES, ids=["x".join(map(str, d)) + f"_k{k}" for d, k in SIZES])
+def test_contractions_at_the_rules_edges(size, fam):
+    L = _lib.lib()
+    dims, K = size
+    ext = dict(zip(("h1", "h2", "h3", "p4", "p5", "p6"), dims), x=K)
+    r = np.random.default_rng(11)
+    names = "h3 h2 h1 p6 p5 p4" + ("" if fam == "s1" else " x")
+    ops = [[k for k in op.split()] for op in OPERANDS[fam]]
+    a, b = (r.standard_normal([ext[k] for k in reversed(op)]) for op in ops)
+    sub = ["".join(LETTER[k] for k in reversed(op)) for op in ops]
+    print(f"percall {fam} {dims} K={K}", flush=True)
+    for n in range(9):
+        layout = (HOLES[fam][n % 3] + " " + PARTICLES[fam][n // 3]).split()
+        out = "".join(LETTER[k] for k in reversed(layout))
+        t3 = r.standard_normal([ext[k] for k in reversed(layout)])
+        eq = f"{sub[0]},{sub[1]}->{out}"
+        want = t3 + SIGN[fam][n] * np.einsum(eq, a, b)
+        bound = (max(K, 1) + 2) * 2.0 ** -53 * np.einsum(eq, np.abs(a), np.abs(b)) + 2.0 ** -52 * np.abs(t3)
+        t3 = np.ascontiguousarray(t3)
+        getattr(L, f"sd_t_{fam}_{n + 1}_")(*refs([ext[k] for k in names.split()]), ptr(t3), ptr(a), ptr(b))
+        assert L.tce_t_legacy_status() == 0, L.tce_t_last_error()
+        assert (np.abs(t3 - want) <= bound).all(), (n + 1, np.abs(t3 - want).max())
