@@ -77,8 +77,8 @@ constexpr int MIXED_MINUS = mixed_minus();
 constexpr int pair_r(int h) { return h == 0 ? 1 : 0; }
 constexpr int pair_s(int h) { return h == 2 ? 1 : 2; }
 
-// Equal boxes of a one-box task (TaskDev::eq): both holes or particles of
-// the pair are the same orbitals.
+// Equal boxes of a work item: both holes or particles of the pair are the same
+// orbitals.
 enum { EQ_IJ = 1, EQ_JK = 2, EQ_AB = 4, EQ_BC = 8 };
 
 struct TaskDev {
@@ -95,7 +95,7 @@ struct TaskDev {
   // h7b / p7b tiles, ccsd_t_doubles_gpu.F:260-263, 924-927); outside it
   // every operand of the pass is zero.  x0 = x1 = 0: no orbital allowed.
   unsigned x[18];
-  int eq;  // EQ_* of a one-box task whose boxes are equal, 0 otherwise
+  int full;  // 1: every element is needed, those of equal boxes too (tile export)
 };
 
 struct FusedArgs {

@@ -192,7 +192,7 @@ __device__ __forceinline__ int particle(const PRange &p, int slot) { return p.g0
 struct ItemGeo {
   HoleBox I, J, K;
   PRange a, b, c;
-  int heq;  // EQ_IJ, EQ_JK of a one-box task
+  int heq;  // EQ_IJ, EQ_JK of the item
   // Whether the pair (u, w) of hole boxes t (0: (j,k), 1: (i,k), 2: (i,j)) has
   // elements that count: inside the boxes, and u < w when the two are one box
   // (the rest follow by antisymmetry, distinct() of them alike).  The epilogue
@@ -231,15 +231,15 @@ __device__ __forceinline__ int cube(int wave, const PRange &p) { return (wave >>
 // lone hole h / lone particle L run; s0 of lone hole h: 1 when the hole pair
 // beside it is one box (its passes form the pairs r < s only).
 struct ItemPlan {
-  int eq;          // TaskDev::eq of a one-box task
+  int eq;          // the item's equal boxes
   int hact, lact;
   __device__ __forceinline__ int s0(int h) const {
     return (h == 2 && (eq & EQ_IJ)) || (h == 0 && (eq & EQ_JK)) ? 1 : 0;
   }
 };
 // half: a half item holds one c half, whose exchange with a or b needs the
-// other, so three equal particle boxes run as two there (the host's tables
-// put a pair of equal boxes on a and b).
+// other, so three equal particle boxes run as two there (the host's one-box
+// tasks put a pair of equal boxes on a and b).
 __device__ __forceinline__ ItemPlan item_plan(int eq, bool half) {
   ItemPlan P;
   if (half && (eq & EQ_AB)) eq &= ~EQ_BC;
@@ -1271,7 +1271,16 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
     G.J = hbox(T->oh2, bj, T->r2);
     G.K = hbox(T->oh3, bk, T->r3);
     auto prng = [](int o, int r, int n) { return PRange{o, min(n - 1, r - 1), 0}; };
-    G.heq = T->eq & (EQ_IJ | EQ_JK);
+    // The item's equal boxes: of the same tile, and of the same place in it
+    // where the tiles hold several (reference tiling).  Reference-tiled jobs used to run all passes of every item:
+    // no=24/nv=120 in tiles of 12 and 40 FP64 184 / 144 ms, FP32 119 / 93, bf16x3
+    // 47.1 / 39.2, bf16x6 68 / 56.
+    int eq = 0;
+    if (EPI != EPI_TILES || !T->full) {  // (read by every kernel, the flag cost 2% of no=40/nv=160)
+      eq = (T->oh1 == T->oh2 && bi == bj ? EQ_IJ : 0) | (T->oh2 == T->oh3 && bj == bk ? EQ_JK : 0);
+      if (T->op4 == T->op5 && ba == bb) eq |= EQ_AB | (T->op5 == T->op6 && bb == bc ? EQ_BC : 0);
+    }
+    G.heq = eq & (EQ_IJ | EQ_JK);
     G.a = prng(T->op4 + 8 * ba, T->r4 - 8 * ba, 8);
     G.b = prng(T->op5 + 8 * bb, T->r5 - 8 * bb, 8);
     G.c = prng(T->op6 + 8 * bc + c4, T->r6 - 8 * bc - c4, HALF ? 4 : 8);
@@ -1291,7 +1300,7 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
         G.a.bit = wa ? (wc ? 1 : 0) + (wb ? 1 : 0) : nw + (wc ? 0 : 1) + (wb ? 0 : 1);
       }
     }
-    const ItemPlan P = item_plan(T->eq, HALF);
+    const ItemPlan P = item_plan(eq, HALF);
     const long part = item * 8 + c4 + wave;  // the wave's partial
 
     double *epi = reinterpret_cast<double *>(lds);

@@ -255,8 +255,7 @@ struct ClassRanges {
 // particle boxes and their hole boxes in descending order of size: t3 t3 / D
 // and t3 y3 / D do not depend on the order, and fused_triples_mixed wastes no
 // MFMA on short second and third boxes (quads past an edge are skipped; the
-// first hole box is the MFMA row index and always counts 4).  TaskDev::eq
-// names the equal boxes.
+// first hole box is the MFMA row index and always counts 4).
 static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool whole,
                         std::vector<TaskDev> &tasks, std::vector<long> &bound,
                         std::vector<long> *task_tiles) {
@@ -276,7 +275,7 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
     if (x[k[1]].r < x[k[2]].r) std::swap(k[1], k[2]);
     if (x[k[0]].r < x[k[1]].r) std::swap(k[0], k[1]);
   };
-  // Fills the boxes, their equalities and the contraction ranges of a one-box
+  // Fills the boxes and the contraction ranges of a one-box
   // task of tiles t6; `have` caches the ranges by box order within a task.
   struct Ranges {
     bool set = false;
@@ -297,8 +296,6 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
     d.r4 = p[kp[0]].r, d.r5 = p[kp[1]].r, d.r6 = p[kp[2]].r;
     d.r1 = h[kh[0]].r, d.r2 = h[kh[1]].r, d.r3 = h[kh[2]].r;
     d.nb4 = d.nb5 = d.nb6 = d.nb1 = d.nb2 = d.nb3 = 1;
-    d.eq = (d.oh1 == d.oh2 ? EQ_IJ : 0) | (d.oh2 == d.oh3 ? EQ_JK : 0) |
-           (d.op4 == d.op5 ? EQ_AB : 0) | (d.op5 == d.op6 ? EQ_BC : 0);
     Ranges &r = have[(kp[0] * 3 + kp[1]) * 9 + kh[0] * 3 + kh[1]];
     if (!r.set) {
       const long t[6] = {t6[kp[0]], t6[kp[1]], t6[kp[2]], t6[3 + kh[0]], t6[3 + kh[1]], t6[3 + kh[2]]};
@@ -306,6 +303,7 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
       r.set = true;
     }
     std::copy(r.d.x, r.d.x + 18, d.x);
+    d.full = 0;
   };
   // sub-tiles of tile b with edge e (the last one ragged)
   auto pieces = [&](long b, int e, bool hole) {
@@ -361,7 +359,7 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
                   d.nb1 = (d.r1 + 3) / 4;
                   d.nb2 = (d.r2 + 3) / 4;
                   d.nb3 = (d.r3 + 3) / 4;
-                  d.eq = 0;
+                  d.full = 0;
                   cr.set(T, tiles6, d);
                 }
                 d.item0 = item;
@@ -1326,6 +1324,7 @@ int tce_t::tile_export_device(Job &J, int precision, long h1b, long h2b, long h3
   d.nb3 = (d.r3 + 3) / 4;
   d.item0 = 0;
   d.factor = 1.0;
+  d.full = 1;
   {
     const long tiles6[6] = {p4b, p5b, p6b, h1b, h2b, h3b};
     ClassRanges(T, J.whole).set(T, tiles6, d);
