@@ -78,7 +78,8 @@ constexpr int pair_r(int h) { return h == 0 ? 1 : 0; }
 constexpr int pair_s(int h) { return h == 2 ? 1 : 2; }
 
 // Equal boxes of a work item: both holes or particles of the pair are the same
-// orbitals.
+// orbitals.  EQ_BC stands beside EQ_AB only (one-box tasks have a pair of equal
+// particle boxes on a and b; elsewhere b == c alone runs as three boxes).
 enum { EQ_IJ = 1, EQ_JK = 2, EQ_AB = 4, EQ_BC = 8 };
 
 struct TaskDev {

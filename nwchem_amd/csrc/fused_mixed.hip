@@ -244,9 +244,9 @@ __device__ __forceinline__ ItemPlan item_plan(int eq, bool half) {
   ItemPlan P;
   if (half && (eq & EQ_AB)) eq &= ~EQ_BC;
   P.eq = eq;
-  const bool ij = eq & EQ_IJ, jk = eq & EQ_JK, ab = eq & EQ_AB, bc = eq & EQ_BC;
+  const bool ij = eq & EQ_IJ, jk = eq & EQ_JK, ab = eq & EQ_AB, bc = eq & EQ_BC;  // bc: all three
   P.hact = ij ? (jk ? 4 : 6) : (jk ? 3 : 7);  // k | j, k | i, j | all
-  P.lact = ab ? (bc ? 4 : 6) : (bc ? 5 : 7);  // c | b, c | a, c | all
+  P.lact = ab ? (bc ? 4 : 6) : 7;             // c | b, c | all
   return P;
 }
 
@@ -622,10 +622,9 @@ __device__ __forceinline__ void chunk_loop(typename Prec<PREC>::quad (&q)[16], c
   }
 }
 
-// Subtracts the partner elements from the accumulators: with x' the element
-// of the exchanged particles (two exchanges when all boxes are equal), q =
-// q - q(a <-> b), q - q(b <-> c), or q - q(a <-> c) - q(b <-> c).  Through LDS
-// in rounds of 64 KB.  A half item has equal boxes a and b only.  Layout c: lane = 4a' + b' + 16c'.
+// Subtracts the partner elements from the accumulators: q - q(a <-> b), or with
+// three equal boxes q - q(a <-> c) - q(b <-> c).  Through LDS in rounds of 64 KB.
+// A half item has equal boxes a and b only.  Layout c: lane = 4a' + b' + 16c'.
 template <int PREC>
 __device__ __forceinline__ void exchange_particles(typename Prec<PREC>::quad (&q)[16], f4 *lds,
                                                    const ItemGeo &G, int eq, int wave, int lane_) {
@@ -635,11 +634,11 @@ __device__ __forceinline__ void exchange_particles(typename Prec<PREC>::quad (&q
   const int a = (lane & 15) >> 2, b = lane & 3, c = lane >> 4;
   const int ca = cube(wave, G.a), cb = cube(wave, G.b), cc = cube(wave, G.c);
   auto from = [&](int x, int y, int z) { return (x << G.a.bit) | (y << G.b.bit) | (z << G.c.bit); };
-  const bool all = (eq & EQ_AB) && (eq & EQ_BC);
+  const bool all = eq & EQ_BC;
   int w1, l1, w2 = 0, l2 = 0;
-  if (eq & EQ_BC) {
+  if (all) {
     w1 = from(ca, cc, cb), l1 = 4 * a + c + 16 * b;
-    if (all) w2 = from(cc, cb, ca), l2 = 4 * c + b + 16 * a;
+    w2 = from(cc, cb, ca), l2 = 4 * c + b + 16 * a;
   } else {
     w1 = from(cb, ca, cc), l1 = 4 * b + a + 16 * c;
   }
@@ -774,14 +773,14 @@ __device__ __forceinline__ void contract(typename Prec<PREC>::quad (&q)[16], f4 
     if (!(P.lact >> L & 1)) continue;
     if (lay >= 0) {
       // a -> b: lane (4b'+c') + 16a' -> (4a'+c') + 16b'; b -> c: (4a'+c') +
-      // 16b' -> (4a'+b') + 16c'; a -> c
+      // 16b' -> (4a'+b') + 16c'
       const int ln = again(lane), kq = ln >> 4, hi = (ln & 15) >> 2, lo = ln & 3;
-      const int src = L == 1 ? 4 * kq + lo + 16 * hi
-                             : (lay == 1 ? 4 * hi + kq + 16 * lo : 4 * lo + kq + 16 * hi);
+      const int src = L == 1 ? 4 * kq + lo + 16 * hi : 4 * hi + kq + 16 * lo;
       permute_lanes(q, src);
     }
     // the passes of a lone particle beside a pair of equal boxes count half:
-    // the exchange at the end adds their image
+    // the exchange at the end adds their image (three equal boxes: c alone runs,
+    // and counts whole)
     const bool half = (P.eq & EQ_BC) ? (L == 0) : ((P.eq & EQ_AB) && L == 2);
     if (half) scale<false, false>(q, (acc)2);
     // lone hole j, then i on the transposed quads
