@@ -226,7 +226,7 @@ struct ClassRanges {
       else l = std::min(l, o), h = std::max(h, e);
     }
   }
-  void set(const Tiles &T, const long tiles[6], TaskDev &d) const {
+  void set(const Tiles &T, const long tiles[6], unsigned (&x)[18]) const {
     for (int p = 0; p < 18; ++p) {
       const PassDef &q = MIXED_PASS[p];
       const long L = tiles[q.L], r = tiles[3 + pair_r(q.h)], s = tiles[3 + pair_s(q.h)];
@@ -234,10 +234,10 @@ struct ClassRanges {
       const int sp = q.kind == 1 ? 0 : 1;
       const bool ok = spin >= 0 && spin <= 3 && sym >= 0 && sym <= 7;
       if (whole) {
-        d.x[p] = (unsigned)(sp ? T.nv : T.no) << 16;
+        x[p] = (unsigned)(sp ? T.nv : T.no) << 16;
         continue;
       }
-      d.x[p] = ok ? (unsigned)lo[sp][spin][sym] | (unsigned)hi[sp][spin][sym] << 16 : 0;
+      x[p] = ok ? (unsigned)lo[sp][spin][sym] | (unsigned)hi[sp][spin][sym] << 16 : 0;
     }
   }
 };
@@ -275,14 +275,18 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
     if (x[k[1]].r < x[k[2]].r) std::swap(k[1], k[2]);
     if (x[k[0]].r < x[k[1]].r) std::swap(k[0], k[1]);
   };
-  // Fills the boxes and the contraction ranges of a one-box
-  // task of tiles t6; `have` caches the ranges by box order within a task.
+  // Fills the boxes and the contraction ranges of a one-box task of tiles t6;
+  // `have` keeps the ranges of the current reference task by box order.  (Made
+  // anew for each reference task, 15 KB, it took a third to half of the plan of
+  // many small tiles: no=20/nv=80 in tiles of 2 and 6 110 ms, now 57; in
+  // orbital tiling 2.3 and 1.1.)
   struct Ranges {
-    bool set = false;
-    TaskDev d;
+    size_t task = 0;  // reference tasks counted from 1
+    unsigned x[18];
   };
+  std::vector<Ranges> have(81);
   auto one_box_task = [&](TaskDev &d, const long (&t6)[6], const Piece (&p)[3],
-                          const Piece (&h)[3], std::vector<Ranges> &have) {
+                          const Piece (&h)[3]) {
     int kp[3], kh[3];
     order3(p, kp);
     order3(h, kh);
@@ -297,21 +301,21 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
     d.r1 = h[kh[0]].r, d.r2 = h[kh[1]].r, d.r3 = h[kh[2]].r;
     d.nb4 = d.nb5 = d.nb6 = d.nb1 = d.nb2 = d.nb3 = 1;
     Ranges &r = have[(kp[0] * 3 + kp[1]) * 9 + kh[0] * 3 + kh[1]];
-    if (!r.set) {
+    if (r.task != bound.size()) {
       const long t[6] = {t6[kp[0]], t6[kp[1]], t6[kp[2]], t6[3 + kh[0]], t6[3 + kh[1]], t6[3 + kh[2]]};
-      cr.set(T, t, r.d);
-      r.set = true;
+      cr.set(T, t, r.x);
+      r.task = bound.size();
     }
-    std::copy(r.d.x, r.d.x + 18, d.x);
+    std::copy(r.x, r.x + 18, d.x);
     d.full = 0;
   };
-  // sub-tiles of tile b with edge e (the last one ragged)
-  auto pieces = [&](long b, int e, bool hole) {
-    std::vector<Piece> v;
-    const int o = (int)(T.ofs(b) - (hole ? 0 : T.no)), r = (int)T.rng(b);
-    for (int k = 0; k < r; k += e) v.push_back({o + k, std::min(e, r - k)});
-    return v;
-  };
+  // sub-tiles of every tile, of edge 4 (holes) or pb, the last one ragged
+  std::vector<std::vector<Piece>> pieces(noab + nvab + 1);
+  for (long b = 1; sub && b <= noab + nvab; ++b) {
+    const bool hole = b <= noab;
+    const int o = (int)(T.ofs(b) - (hole ? 0 : T.no)), r = (int)T.rng(b), e = hole ? 4 : pb;
+    for (int k = 0; k < r; k += e) pieces[b].push_back({o + k, std::min(e, r - k)});
+  }
   auto sym_factor = [](bool e12, bool e23) {
     return (e12 && e23) ? 1.0 / 6.0 : ((e12 || e23) ? 0.5 : 1.0);
   };
@@ -333,7 +337,6 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
               if (!task_allowed(T, p4b, p5b, p6b, h1b, h2b, h3b)) continue;
               bound.push_back(item);
               const long tiles6[6] = {p4b, p5b, p6b, h1b, h2b, h3b};
-              std::vector<Ranges> have(81);
               if (task_tiles) {
                 long tt[6] = {p4b, p5b, p6b, h1b, h2b, h3b};
                 task_tiles->insert(task_tiles->end(), tt, tt + 6);
@@ -347,7 +350,7 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
                                     {(int)T.ofs(h2b), (int)T.rng(h2b)},
                                     {(int)T.ofs(h3b), (int)T.rng(h3b)}};
                 if (one_box) {
-                  one_box_task(d, tiles6, p, h, have);
+                  one_box_task(d, tiles6, p, h);
                 } else {
                   d.op4 = p[0].o, d.op5 = p[1].o, d.op6 = p[2].o;
                   d.oh1 = h[0].o, d.oh2 = h[1].o, d.oh3 = h[2].o;
@@ -360,7 +363,7 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
                   d.nb2 = (d.r2 + 3) / 4;
                   d.nb3 = (d.r3 + 3) / 4;
                   d.full = 0;
-                  cr.set(T, tiles6, d);
+                  cr.set(T, tiles6, d.x);
                 }
                 d.item0 = item;
                 d.factor = task_factor(T.restricted, p4b, p5b, p6b, h1b, h2b, h3b);
@@ -368,15 +371,14 @@ static long build_tasks(const Tiles &T, int pb, bool sub, bool one_box, bool who
                 tasks.push_back(d);
                 continue;
               }
-              const auto A = pieces(p4b, pb, false), B = pieces(p5b, pb, false),
-                         C = pieces(p6b, pb, false), I = pieces(h1b, 4, true),
-                         J = pieces(h2b, 4, true), K = pieces(h3b, 4, true);
+              const auto &A = pieces[p4b], &B = pieces[p5b], &C = pieces[p6b], &I = pieces[h1b],
+                         &J = pieces[h2b], &K = pieces[h3b];
               const bool pab = p4b == p5b, pbc = p5b == p6b, hij = h1b == h2b, hjk = h2b == h3b;
               const double rf = T.restricted ? 2.0 : 1.0;
               auto emit = [&](size_t a, size_t b, size_t c, size_t i, size_t j, size_t k) {
                 TaskDev d;
                 const Piece p[3] = {A[a], B[b], C[c]}, h[3] = {I[i], J[j], K[k]};
-                one_box_task(d, tiles6, p, h, have);
+                one_box_task(d, tiles6, p, h);
                 d.item0 = item++;
                 d.factor = rf * sym_factor(hij && i == j, hjk && j == k) *
                            sym_factor(pab && a == b, pbc && b == c);
@@ -1327,7 +1329,7 @@ int tce_t::tile_export_device(Job &J, int precision, long h1b, long h2b, long h3
   d.full = 1;
   {
     const long tiles6[6] = {p4b, p5b, p6b, h1b, h2b, h3b};
-    ClassRanges(T, J.whole).set(T, tiles6, d);
+    ClassRanges(T, J.whole).set(T, tiles6, d.x);
   }
   const long n = (long)d.r1 * d.r2 * d.r3 * d.r4 * d.r5 * d.r6;
   const long items = (long)d.nb4 * d.nb5 * d.nb6 * d.nb1 * d.nb2 * d.nb3;
