@@ -271,16 +271,16 @@ struct Runs {
 
 // Host ranges to the device.  The referenced ranges of a file form one stream
 // of R.total doubles (the runs in order, at device offsets base[k]); the
-// streams are cut into pieces.  Up to 256 MiB in all (small()), the pieces are of
+// streams are cut into pieces.  Up to 384 MiB in all (small()), the pieces are of
 // 1 MiB and the host threads take them in turn: each gathers a piece into one
 // of its two pinned buffers and queues that buffer's copy, so gathers and DMA
 // overlap throughout and the pinned memory, 32 MiB at most, stays in the host's
 // caches.  Above, all threads together gather a piece of 64 MiB into one of two
-// pinned buffers while the DMA of the other runs (large()).  Measured at 74 MB
-// (no=20/nv=80, DMA alone 1.5 ms): large 7.7 ms, of which threads started for
-// each buffer and the pinning of 128 MiB take half, small 3.7; no=8/nv=32 2.2
-// and 0.5 ms; at 1.9 GB (no=40/nv=160), where the DMA bounds both, large 38 ms,
-// small 45 (copies of 4 MiB 40, 8 MiB 41).
+// pinned buffers while the DMA of the other runs (large()).  Upload of a job,
+// large / small: 2 MB 2.2 / 0.4 ms, 74 MB 8.5 / 4.2 (threads started for each
+// buffer and the pinning of 128 MiB take half of the 8.5; the DMA alone 1.5), 185
+// MB 13.4 / 10.0, 300 MB 16.6 / 13.0, 426 MB 19.8 / 20.3, 615 MB 24 / 26, 1.2 GB
+// 38 / 48.  (large() with a thread for each piece only: 15 ms at 74 MB, 21 at 300.)
 class Upload {
  public:
   Upload(int device, hipStream_t stream, char *dst) : device_(device), stream_(stream), dst_(dst) {}
@@ -304,7 +304,8 @@ class Upload {
         pieces_.push_back({f.R, f.file, p, std::min(piece_, f.n - p), f.at + (size_t)p * sizeof(double)});
     const long np = (long)pieces_.size();
     if (np == 0) return hipSuccess;
-    const long nt = std::min({np, 16l, std::max(1l, (long)std::thread::hardware_concurrency())});
+    const long hw = std::min(16l, std::max(1l, (long)std::thread::hardware_concurrency()));
+    const long nt = total <= SMALL ? std::min(np, hw) : hw;
     const long slots = total <= SMALL ? std::min(np, 2 * nt) : 2;
     hipError_t e = hipHostMalloc((void **)&stage_, slots * piece_ * sizeof(double));
     for (long k = 0; k < slots && e == hipSuccess; ++k) {
@@ -317,7 +318,7 @@ class Upload {
   }
 
  private:
-  static constexpr long SMALL = 1l << 25;  // doubles
+  static constexpr long SMALL = 3l << 24;  // doubles
   struct Piece {
     const Runs *R;
     const double *file;
