@@ -184,15 +184,21 @@ int lambda_fused(Job &JR, Job &JL, const double *dF, int precision, std::vector<
   if (N > 0) {
     int cus = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, JR.device), "attr");
-    const int grid = (int)std::min<long>(std::max(1, cus), N);
-    const size_t need =
-        (size_t)grid * pair_slot_doubles(cr_den != nullptr, precision != TCE_T_FP64) * sizeof(double);
-    if (JR.dspill_bytes < need) {
+    int grid = (int)std::min<long>(std::max(1, cus), N);
+    const size_t slot =
+        pair_slot_doubles(cr_den != nullptr, precision != TCE_T_FP64) * sizeof(double);
+    if (JR.dspill_bytes < grid * slot) {
       if (JR.dspill) HIPCHK(hipFree(JR.dspill), "spill slots");
       JR.dspill = nullptr;
       JR.dspill_bytes = 0;
-      HIPCHK(hipMalloc(&JR.dspill, need), "spill slots");
-      JR.dspill_bytes = need;
+      // where the device lacks the room for all, fewer workgroups
+      hipError_t e;
+      while ((e = hipMalloc(&JR.dspill, grid * slot)) == hipErrorOutOfMemory && grid > 1) {
+        (void)hipGetLastError();
+        grid = (grid + 1) / 2;
+      }
+      HIPCHK(e, "spill slots");
+      JR.dspill_bytes = grid * slot;
     }
     MixedArgs ML = job_margs(JL, precision), MR = job_margs(JR, precision);
     ML.lam_f = dF;
