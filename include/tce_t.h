@@ -200,7 +200,7 @@ int tce_t_device_memory(long *free_bytes, long *total_bytes);
 int tce_t_job_create(const tce_t_tiles *tiles, tce_t_job **job);
 /* Tiling of the kernel tasks (no reference counterpart; the energies are
  * the same sums, up to FP64 rounding, in every mode):
- *   REFERENCE  the reference tiles, boxes over each (the reference's work);
+ *   REFERENCE  the reference tiles, boxes over each (the reference's elements);
  *   SUBTILE    box-sized sub-tiles of each reference tile (4 occupied, 4 or
  *              8 virtual orbitals) in canonical order: no symmetric
  *              duplicates inside equal tiles; per-task energies and restart

@@ -66,10 +66,10 @@
 // unrolled it was 84 KB, more than the 64 KB instruction cache two CUs share,
 // and every item ran from L2.
 //
-// Together (ms before / after): no=40/nv=160 FP64 635 / 462, no=21/nv=160 in
+// Together (ms before / after): no=40/nv=160 FP64 635 / 460, no=21/nv=160 in
 // ragged tiles 149 / 79, no=26/nv=114 in spin-labelled ragged tiles 17.7 /
-// 5.7, no=40/nv=320 in 2 spins x 4 irreps (tiles of 5 holes) 446 / 185,
-// bf16x6 no=40/nv=200 526 / 456.
+// 5.6, no=40/nv=320 in 2 spins x 4 irreps (tiles of 5 holes) 446 / 186,
+// bf16x6 no=40/nv=200 530 / 450.
 //
 // LDS layout of one buffer part (hi or lo; quads, kq = quad 0..3 of a row):
 //   X  [4 s][8 L slots][4 r][4 kq ^ x_swz]         512 quads
@@ -1271,9 +1271,9 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
     G.K = hbox(T->oh3, bk, T->r3);
     auto prng = [](int o, int r, int n) { return PRange{o, min(n - 1, r - 1), 0}; };
     // The item's equal boxes: of the same tile, and of the same place in it
-    // where the tiles hold several (reference tiling).  Reference-tiled jobs used to run all passes of every item:
-    // no=24/nv=120 in tiles of 12 and 40 FP64 184 / 144 ms, FP32 119 / 93, bf16x3
-    // 47.1 / 39.2, bf16x6 68 / 56.
+    // where the tiles hold several (reference tiling).  Told per task, they served
+    // one-box tasks only; reference-tiled no=24/nv=120 in tiles of 12 and 40 then
+    // and now: FP64 184 / 144 ms, FP32 119 / 93, bf16x3 47.1 / 39.2, bf16x6 68 / 56.
     int eq = 0;
     if (EPI != EPI_TILES || !T->full) {  // (read by every kernel, the flag cost 2% of no=40/nv=160)
       eq = (T->oh1 == T->oh2 && bi == bj ? EQ_IJ : 0) | (T->oh2 == T->oh3 && bj == bk ? EQ_JK : 0);
@@ -1321,8 +1321,8 @@ __global__ void __launch_bounds__(64 * Prec<PREC>::NW, 2) fused_triples_mixed(co
     // half items: 134 us, now 104), and the last round of a longer one was less
     // even (CR no=16/nv=72 4.76 / 4.61 ms, Lambda no=20/nv=80 15.3 / 15.2).
     // (The order of the tests here and below is the faster one of each kernel, all
-    // of which sit at the register limit: `dyn` first, no=40/nv=160 461 ms and a
-    // tile export of no=24/nv=96 1.28 ms; `dyn` second, 465 and 1.18 ms.)
+    // of which sit at the register limit: `dyn` first, no=40/nv=160 460 ms and a
+    // tile export of no=24/nv=96 1.30 ms; `dyn` second, 465 and 1.17 ms.)
     if (EPI == EPI_TILES ? empty && dyn && tid == 0 : dyn && empty && tid == 0)
       ticket = atomicAdd(&sched[queue], 1ull);
     if (empty && EPI != EPI_TILES && lane == 0) {

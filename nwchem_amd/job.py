@@ -24,7 +24,7 @@ BF16X3 = 2  # operands split into bf16 hi + lo, hi*hi + hi*lo + lo*hi, FP32 accu
 BF16X6 = 3  # operands split into bf16 hi + mid + lo, the 6 products to 2^-24, FP32 accumulation
 
 # Kernel-task tilings (tce_t_job_create_tiling)
-TILING_REFERENCE = 0  # the reference tiles (the reference's work)
+TILING_REFERENCE = 0  # the reference tiles (the reference's elements)
 TILING_SUBTILE = 1    # box-sized sub-tiles of each reference tile (default)
 TILING_ORBITAL = 2    # box-sized pieces of each spin/irrep run of orbitals; totals only
 
