@@ -909,20 +909,12 @@ __device__ __forceinline__ void each_element(const ItemGeo &G, double (&v)[64], 
 // no=16/nv=72, of which the kernels took 45 and 7.7 ms) and two passes over it
 // in HBM.
 // What the slots cost is not their own time but the operands they push out of
-// the caches: with 64-bit doubles and ordinary accesses a CR item's bf16x3
-// contractions at no=40/nv=160 took 258k clocks a side, 186k without the slot
-// accesses (the FP64 mode's, 742k, change by 1%).  FP32 doubles bring 193k, and
-// accesses marked as streaming 187k.  CR before / now (two launches over a
-// window), s: bf16x3 no=40/nv=160 0.351 / 0.275 (0.333), no=40/nv=320 4.19 / 3.34
-// (3.60); bf16x6 0.486 / 0.419 (0.509) and 6.14 / 5.47 (5.97).
-template <class T, class V>
-__device__ __forceinline__ void slot_put(gptr<T> slot, int r, int lane, V v) {
-  __builtin_nontemporal_store((T)v, &slot[r * 64 + lane]);
-}
-template <class T>
-__device__ __forceinline__ T slot_get(gptr<const T> slot, int r, int lane) {
-  return __builtin_nontemporal_load(&slot[r * 64 + lane]);
-}
+// the caches: with 64-bit doubles a CR item's bf16x3 contractions at no=40/nv=160
+// took 258k clocks a side, 186k without the slot accesses (the FP64 mode's, 742k,
+// change by 1%), with FP32 doubles they take 193k.  CR before / now (two launches
+// over a window), s: bf16x3 no=40/nv=160 0.351 / 0.276 (0.333), no=40/nv=320 4.19 /
+// 3.37 (3.60); bf16x6 0.486 / 0.422 (0.509) and 6.19 / 5.47 (5.97).  Accesses marked
+// as streaming: 2% faster there, 1 to 2% slower at no=16/nv=72 in FP64 and FP32.
 // The CR doubles' type in the slot, and the singles' place behind them.
 template <class Q>
 using slot_t = std::conditional_t<sizeof(Q) == 16, float, double>;
@@ -942,7 +934,7 @@ __device__ __forceinline__ void each_element_with(const ItemGeo &G, gptr<const d
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
       v[16 * (n >> 2) + 4 * jj + (n & 3)] = 0.0;
-      x[n] = slot_get(in, 16 * (n >> 2) + 4 * jj + (n & 3), lane);
+      x[n] = in[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
     }
     if (jj < G.J.n)
 #pragma unroll
@@ -1068,7 +1060,7 @@ __device__ __forceinline__ void lambda_left(const Q (&q)[16], const double *e, b
   for (int r = 0; r < 64; ++r) yd[r] = (double)q[r & 15][r >> 4];
   if (fock) each_single(e, G, p, [&](int r, double s) { yd[r] += s; });
 #pragma unroll
-  for (int r = 0; r < 64; ++r) slot_put(out, r, lane, yd[r]);
+  for (int r = 0; r < 64; ++r) out[r * 64 + lane] = yd[r];
 }
 
 // Left-hand half of a CR item: the t3 doubles and singles.
@@ -1076,12 +1068,12 @@ template <class Q>
 __device__ __forceinline__ void cr_left(const Q (&q)[16], const double *e, const Place &p,
                                         const ItemGeo &G, gptr<double> out, int lane) {
 #pragma unroll
-  for (int r = 0; r < 64; ++r) slot_put((gptr<slot_t<Q>>)out, r, lane, q[r & 15][r >> 4]);
+  for (int r = 0; r < 64; ++r) ((gptr<slot_t<Q>>)out)[r * 64 + lane] = q[r & 15][r >> 4];
   phase();
   double sv[64];
   singles_products(e, G, p, sv);
 #pragma unroll
-  for (int r = 0; r < 64; ++r) slot_put(out + singles_at<slot_t<Q>>(), r, lane, sv[r]);
+  for (int r = 0; r < 64; ++r) out[singles_at<slot_t<Q>>() + r * 64 + lane] = sv[r];
 }
 
 // Right-hand half of a Lambda item: den = t3d * factor / D as in energy(), e1
@@ -1147,8 +1139,8 @@ __device__ __forceinline__ void cr_right(const Q (&q)[16], const double *e, cptr
 #pragma unroll
         for (int n = 0; n < 8; ++n) {
           const int r = 16 * (i0 + (n >> 2)) + 4 * jj + (n & 3);
-          td[n] = slot_get(in1, r, lane);
-          ts[n] = slot_get(in2, r, lane);
+          td[n] = in1[r * 64 + lane];
+          ts[n] = in2[r * 64 + lane];
         }
         if (jj < G.J.n)
 #pragma unroll
@@ -1177,8 +1169,8 @@ __device__ __forceinline__ void cr_right(const Q (&q)[16], const double *e, cptr
     double td[16], ts[16];
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
-      td[n] = slot_get(in, 16 * (n >> 2) + 4 * jj + (n & 3), lane);
-      ts[n] = slot_get(ins, 16 * (n >> 2) + 4 * jj + (n & 3), lane);
+      td[n] = in[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
+      ts[n] = ins[(16 * (n >> 2) + 4 * jj + (n & 3)) * 64 + lane];
     }
     if (jj < G.J.n)
 #pragma unroll
